@@ -307,25 +307,7 @@ hipError_t launch_grad_contract(const NvOpDev &g, const double *ub, const double
     }
 }
 
-// ---- broadened spectrum of the tridiagonal eigenpairs -------------------------
-// env[g] = sum_i a_i^2 G(grid[g] - (theta_i - ref) c),  a_i = vec[i] (first
-// components), G(u) = exp(-u^2 / (2 sigma^2)).
-__global__ __launch_bounds__(256) void spec_env_kernel(int64_t n, const double *__restrict__ theta,
-                                                      const double *__restrict__ vec, double ref, double c,
-                                                      double sigma, int64_t ng, const double *__restrict__ grid,
-                                                      double *__restrict__ env) {
-    const int64_t gi = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (gi >= ng) return;
-    const double x = grid[gi];
-    double s = 0.0;
-    for (int64_t i = 0; i < n; ++i) {
-        const double a = vec[i];
-        const double u = (x - (theta[i] - ref) * c) / sigma;
-        s = fma(a * a, exp(-0.5 * u * u), s);
-    }
-    env[gi] = s;
-}
-
+// ---- adjoint of the broadened spectrum (its forward pass is in nv_spectrum.hip) ----
 // W[i] = sum_g gbar_g G(u_gi), Wp[i] = sum_g gbar_g u_gi G(u_gi) c / sigma: one block per root.
 __global__ __launch_bounds__(256) void spec_w_kernel(const double *__restrict__ theta, double ref, double c,
                                                     double sigma, int64_t ng, const double *__restrict__ grid,
@@ -457,12 +439,6 @@ __global__ __launch_bounds__(256) void spec_rows_kernel(int64_t n, const double 
         abar[j] = d;
         if (j + 1 < n) bbar[j + 1] = 2.0 * o;
     }
-}
-
-hipError_t launch_spec_env(int64_t n, const double *theta, const double *vec, double ref, double c, double sigma,
-                           int64_t ng, const double *grid, double *env, hipStream_t s) {
-    spec_env_kernel<<<(unsigned)((ng + 255) / 256), 256, 0, s>>>(n, theta, vec, ref, c, sigma, ng, grid, env);
-    return hipGetLastError();
 }
 
 hipError_t launch_spec_adjoint(int64_t n, const double *theta, const double *vec, double ref, int lowest, double c,

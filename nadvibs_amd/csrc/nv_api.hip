@@ -77,13 +77,17 @@ struct nv_ctx {
     std::vector<std::pair<hipEvent_t, hipEvent_t>> ev;
     size_t ev_used = 0;
     size_t lz_bytes_key = 0;
+
+    // device workspace of the tridiagonal eigensolve, kept between calls up to kTriKeepBytes
+    void *tri = nullptr;
+    size_t tri_bytes = 0;
 };
 
 static std::string g_create_error;
 
 // ---- static scratch of the no-allocation entry point ------------------------
-// nv_convolve_noalloc keeps its per-workgroup maxima (one double per kBlock grid
-// points) here instead of in an allocation: 32 KiB per GPU, held until the
+// nv_convolve_noalloc keeps its per-workgroup maxima (nv::convolve_parts doubles,
+// at most one per kBlock points of the largest grid) here instead of in an allocation: 32 KiB per GPU, held until the
 // process ends.  In host code `scratch` only names the symbol; its address on
 // each device comes from hipGetSymbolAddress, taken once per device in
 // nv_create with that device current.
@@ -381,6 +385,7 @@ int32_t nv_destroy(nv_ctx *c) {
     if (c->d_startvals) hipFree(c->d_startvals);
     if (c->hx) hipFree(c->hx);
     if (c->hy) hipFree(c->hy);
+    if (c->tri) hipFree(c->tri);
     if (c->stream) hipStreamDestroy(c->stream);
     delete c;
     return NV_OK;
@@ -1094,15 +1099,40 @@ int32_t nv_get_lanczos_vector(nv_ctx *c, int64_t j, double *q) {
 }
 
 // ---- tridiagonal eigensolve ---------------------------------------------
+// The workspace of one eigensolve (5 n^2 doubles, 360 MB at n = 3000) stays with the context, as a
+// program solves again and again while it iterates; a larger one goes back after each call.
+constexpr size_t kTriKeepBytes = (size_t)512 << 20;
+
+static hipError_t tri_reserve(nv_ctx *c, size_t bytes) {
+    if (c->tri_bytes >= bytes) return hipSuccess;
+    if (c->tri) hipFree(c->tri);
+    c->tri = nullptr;
+    c->tri_bytes = 0;
+    hipError_t e = hipMalloc(&c->tri, bytes);
+    if (e == hipSuccess) c->tri_bytes = bytes;
+    else c->tri = nullptr;
+    return e;
+}
+
+// After the last use of an eigensolve's vectors (the stream synchronised).
+static void tri_trim(nv_ctx *c) {
+    if (c->tri_bytes <= kTriKeepBytes) return;
+    hipFree(c->tri);
+    c->tri = nullptr;
+    c->tri_bytes = 0;
+}
+
 // Eigenvalues (ascending) and eigenvectors of the tridiagonal T(alpha,
 // beta(1:n-1)) on the device.  *vec_dev (n*n doubles, vec[j*n + i] =
-// component j of root i) belongs to the caller, who frees it with hipFree.
+// component j of root i) lies in the context's workspace until the next
+// solve; the caller ends with tri_trim.
 static int32_t tridiag_solve(nv_ctx *c, int64_t n, const double *alpha, const double *beta,
                              std::vector<double> &root, double **vec_dev) {
     *vec_dev = nullptr;
     for (int64_t i = 0; i < n; ++i)
         if (!std::isfinite(alpha[i]) || !std::isfinite(beta[i + 1]))
             return fail(c, NV_ERR_ARG, "alpha/beta hold a non-finite value at iteration " + std::to_string(i + 1));
+    if (n > ((int64_t)1 << 30)) return fail(c, NV_ERR_NOMEM, "tridiagonal problem too large");
     NV_HIP(c, hipSetDevice(c->device));
     root.assign(n, 0.0);
     // Frobenius scaling in the order GIVENS accumulates it (Source/yarkony.f90:221-247)
@@ -1111,19 +1141,16 @@ static int32_t tridiag_solve(nv_ctx *c, int64_t n, const double *alpha, const do
         factor = std::fmax(factor, std::fabs(alpha[i]));
         if (i > 0) factor = std::fmax(factor, std::fabs(beta[i]));
     }
-    double *vec = nullptr;
-    NV_HIP(c, hipMalloc(&vec, (size_t)n * n * sizeof(double)));
     if (n == 1 || factor == 0.0) {
+        NV_HIP(c, tri_reserve(c, (size_t)n * n * sizeof(double)));
+        double *vec = (double *)c->tri;
         std::vector<double> eye((size_t)n * n, 0.0);
         for (int64_t i = 0; i < n; ++i) {
             eye[(size_t)i * n + i] = 1.0;
             root[i] = n == 1 ? alpha[0] : 0.0;
         }
         hipError_t er = hipMemcpy(vec, eye.data(), (size_t)n * n * sizeof(double), hipMemcpyHostToDevice);
-        if (er != hipSuccess) {
-            hipFree(vec);
-            return hip_fail(c, er, "tridiagonal eigenvectors");
-        }
+        if (er != hipSuccess) return hip_fail(c, er, "tridiagonal eigenvectors");
         *vec_dev = vec;
         return NV_OK;
     }
@@ -1133,37 +1160,43 @@ static int32_t tridiag_solve(nv_ctx *c, int64_t n, const double *alpha, const do
         anorm += (alpha[i] / factor) * (alpha[i] / factor) / 2.0;
     }
     anorm = std::sqrt(anorm * 2.0) * factor;
-    std::vector<double> d(n), e(n, 0.0), e2(n, 0.0);
-    for (int64_t i = 0; i < n; ++i) d[i] = alpha[i] / anorm;
-    for (int64_t i = 0; i + 1 < n; ++i) { e[i] = beta[i + 1] / anorm; e2[i] = e[i] * e[i]; }
-    nv::TriWork w;
-    w.vec = vec;
-    std::vector<void *> tmp;
-    auto alloc = [&](size_t bytes, void **p) -> hipError_t {
-        hipError_t er = hipMalloc(p, bytes);
-        if (er == hipSuccess) tmp.push_back(*p);
-        return er;
+    // one upload: (d_j, e_{j-1}^2) rows, then d, then e
+    const size_t nde = 2 * ((size_t)n + nv::kTriPad);
+    std::vector<double> up(nde + 2 * (size_t)n, 0.0);
+    double *hde = up.data(), *hd = hde + nde, *he = hd + n;
+    for (int64_t i = 0; i < n; ++i) hde[2 * i] = hd[i] = alpha[i] / anorm;
+    for (int64_t i = 0; i + 1 < n; ++i) {
+        he[i] = beta[i + 1] / anorm;
+        hde[2 * (i + 1) + 1] = std::fmax(he[i] * he[i], nv::kTriMinE2);
+    }
+    size_t at = 0;
+    auto carve = [&](size_t bytes) {
+        const size_t o = at;
+        at += (bytes + 255) & ~(size_t)255;
+        return o;
     };
-    hipError_t er = alloc(n * 8, (void **)&w.d);
-    if (er == hipSuccess) er = alloc(n * 8, (void **)&w.e);
-    if (er == hipSuccess) er = alloc(n * 8, (void **)&w.e2);
-    if (er == hipSuccess) er = alloc(n * 8, (void **)&w.root);
-    if (er == hipSuccess) er = alloc((size_t)4 * n * n * 8, (void **)&w.lu);
-    if (er == hipSuccess) er = alloc(n * 4, (void **)&w.ia);
-    if (er == hipSuccess) er = alloc(n * 8, (void **)&w.rank);
-    if (er == hipSuccess) er = hipMemcpyAsync(w.d, d.data(), n * 8, hipMemcpyHostToDevice, c->stream);
-    if (er == hipSuccess) er = hipMemcpyAsync(w.e, e.data(), n * 8, hipMemcpyHostToDevice, c->stream);
-    if (er == hipSuccess) er = hipMemcpyAsync(w.e2, e2.data(), n * 8, hipMemcpyHostToDevice, c->stream);
-    if (er == hipSuccess) er = nv::launch_tridiag(n, w, anorm, c->stream);
+    const size_t o_vec = carve((size_t)n * n * 8), o_lu = carve((size_t)4 * n * n * 8), o_up = carve(up.size() * 8),
+                 o_root = carve(n * 8), o_rank = carve(n * 8), o_ia = carve(n * 4),
+                 o_cnt = carve((size_t)nv::tri_grid_points(n) * 4);
+    NV_HIP(c, tri_reserve(c, at));
+    char *base = (char *)c->tri;
+    nv::TriWork w;
+    w.vec = (double *)(base + o_vec);
+    w.lu = (double *)(base + o_lu);
+    w.de = (double *)(base + o_up);
+    w.d = w.de + nde;
+    w.e = w.d + n;
+    w.root = (double *)(base + o_root);
+    w.rank = (int64_t *)(base + o_rank);
+    w.ia = (int32_t *)(base + o_ia);
+    w.cnt = (int32_t *)(base + o_cnt);
+    hipError_t er = hipMemcpyAsync(w.de, up.data(), up.size() * 8, hipMemcpyHostToDevice, c->stream);
+    if (er == hipSuccess) er = nv::launch_tridiag(n, w, c->stream);
     if (er == hipSuccess) er = hipMemcpyAsync(root.data(), w.root, n * 8, hipMemcpyDeviceToHost, c->stream);
     if (er == hipSuccess) er = hipStreamSynchronize(c->stream);
-    for (void *p : tmp) hipFree(p);
-    if (er != hipSuccess) {
-        hipFree(vec);
-        return hip_fail(c, er, "tridiagonal eigensolve");
-    }
+    if (er != hipSuccess) return hip_fail(c, er, "tridiagonal eigensolve");
     for (int64_t i = 0; i < n; ++i) root[i] *= anorm;
-    *vec_dev = vec;
+    *vec_dev = w.vec;
     return NV_OK;
 }
 
@@ -1178,7 +1211,7 @@ int32_t nv_ritz(nv_ctx *c, int64_t n, const double *alpha, const double *beta, d
     hipError_t er = hipMemcpyAsync(v1.data(), vec, n * 8, hipMemcpyDeviceToHost, c->stream);
     if (er == hipSuccess) er = hipMemcpyAsync(vn.data(), vec + (n - 1) * n, n * 8, hipMemcpyDeviceToHost, c->stream);
     if (er == hipSuccess) er = hipStreamSynchronize(c->stream);
-    hipFree(vec);
+    tri_trim(c);
     if (er != hipSuccess) return hip_fail(c, er, "tridiagonal eigenvectors");
     const double bn = beta[n];
     for (int64_t i = 0; i < n; ++i) {
@@ -1211,7 +1244,7 @@ int32_t nv_identify_roots(nv_ctx *c, int64_t n, const double *alpha, const doubl
     double *vec = nullptr;
     int32_t rc = tridiag_solve(c, n, alpha, beta, root, &vec);
     if (rc != NV_OK) return rc;
-    std::vector<void *> tmp{vec};
+    std::vector<void *> tmp;
     auto alloc = [&](size_t bytes, void **p) -> hipError_t {
         hipError_t er = hipMalloc(p, bytes);
         if (er == hipSuccess) tmp.push_back(*p);
@@ -1257,6 +1290,7 @@ int32_t nv_identify_roots(nv_ctx *c, int64_t n, const double *alpha, const doubl
         er = hipMemcpyAsync(vectors, Y, (size_t)nroots * N * 8, hipMemcpyDeviceToHost, c->stream);
     if (er == hipSuccess) er = hipStreamSynchronize(c->stream);
     for (void *p : tmp) hipFree(p);
+    tri_trim(c);
     if (er != hipSuccess) return hip_fail(c, er, "identify_roots");
     // intensities relative to the strongest of the nroots roots (Source/top.f90:1165-1168)
     double intfactor = 0.0;
@@ -1524,7 +1558,7 @@ static int32_t spectrum_common(nv_ctx *c, int64_t n, const double *alpha, const 
     double *vec = nullptr;
     int32_t rc = tridiag_solve(c, n, alpha, beta, root, &vec);
     if (rc != NV_OK) return rc;
-    std::vector<void *> tmp{vec};
+    std::vector<void *> tmp;
     auto alloc = [&](size_t bytes, void **p) -> hipError_t {
         hipError_t er = hipMalloc(p, bytes);
         if (er == hipSuccess) tmp.push_back(*p);
@@ -1559,6 +1593,7 @@ static int32_t spectrum_common(nv_ctx *c, int64_t n, const double *alpha, const 
     }
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     for (void *p : tmp) hipFree(p);
+    tri_trim(c);
     if (e != hipSuccess) return hip_fail(c, e, "spectrum");
     return NV_OK;
 }
@@ -1719,9 +1754,8 @@ int32_t nv_convolve(nv_ctx *c, int64_t n, const double *x, const double *y, int6
     if (n < 1 || ng < 1 || !x || !y || !grid || !env || !(sigma > 0))
         return fail(c, NV_ERR_ARG, "bad convolve arguments");
     NV_HIP(c, hipSetDevice(c->device));
-    const int nb = (int)((ng + nv::kBlock - 1) / nv::kBlock);
     double *d = nullptr;
-    const size_t bytes = (size_t)(2 * n + 2 * ng + nb) * sizeof(double);
+    const size_t bytes = (size_t)(2 * n + 2 * ng + nv::convolve_parts(ng)) * sizeof(double);
     NV_HIP(c, hipMalloc(&d, bytes));
     double *dx = d, *dy = d + n, *dg = d + 2 * n, *de = d + 2 * n + ng, *dp = d + 2 * n + 2 * ng;
     hipError_t e = hipMemcpyAsync(dx, x, n * 8, hipMemcpyHostToDevice, c->stream);

@@ -9,8 +9,6 @@
 //                  dots reduced to per-block partials and summed by a
 //                  one-block finish kernel (fixed summation order:
 //                  reproducible run to run).
-//  * tri_*         Sturm bisection and inverse iteration for the tridiagonal
-//                  eigenproblem, one root per thread.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -2137,58 +2135,6 @@ hipError_t launch_norm_to(const double *v, int64_t n, double *out, double *parti
     return launch_finish_sum(partials, g, out, nullptr, 1, s);
 }
 
-// ------------------------------------------------------------------------
-// Gaussian broadening of a stick spectrum (convolve.py:28-48):
-// env[g] = sum_j y_j exp(-((grid_g - x_j)/sigma)^2 / 2), then env / max(env).
-// One thread per grid point; the sticks are staged through LDS in tiles.
-// ------------------------------------------------------------------------
-__global__ __launch_bounds__(kBlock) void convolve_kernel(const double *x, const double *y, int64_t n,
-                                                          const double *grid, int64_t ng, double sigma, double *env,
-                                                          double *part) {
-    __shared__ double sx[kBlock], sy[kBlock];
-    const int64_t g = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    const double gx = g < ng ? grid[g] : 0.0;
-    const double inv = 1.0 / sigma;
-    double acc = 0.0;
-    for (int64_t j0 = 0; j0 < n; j0 += kBlock) {
-        __syncthreads();
-        if (j0 + threadIdx.x < n) {
-            sx[threadIdx.x] = x[j0 + threadIdx.x];
-            sy[threadIdx.x] = y[j0 + threadIdx.x];
-        }
-        __syncthreads();
-        const int m = (int)(n - j0 < kBlock ? n - j0 : kBlock);
-        for (int j = 0; j < m; ++j) {
-            const double t = (gx - sx[j]) * inv;
-            acc += sy[j] * exp(-0.5 * t * t);
-        }
-    }
-    if (g < ng) env[g] = acc;
-    // block maximum for the normalisation
-    double mx = g < ng ? acc : -INFINITY;
-    for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off, 64));
-    __shared__ double red[kBlock / 64];
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double m2 = red[0];
-        for (int w = 1; w < kBlock / 64; ++w) m2 = fmax(m2, red[w]);
-        part[blockIdx.x] = m2;
-    }
-}
-
-__global__ __launch_bounds__(kBlock) void convolve_norm_kernel(double *env, int64_t ng, const double *part, int nb) {
-    __shared__ double mx;
-    if (threadIdx.x == 0) {
-        double m = part[0];
-        for (int b = 1; b < nb; ++b) m = fmax(m, part[b]);
-        mx = m;
-    }
-    __syncthreads();
-    for (int64_t g = (int64_t)blockIdx.x * kBlock + threadIdx.x; g < ng; g += (int64_t)gridDim.x * kBlock)
-        env[g] /= mx;
-}
-
 // Overlaps of up to kMaxProbes probe vectors with basis vectors j0..j0+nj-1
 // (q_j in slot j % nslots of V): grid (chunks, nj), partial dots per chunk in
 // part[(k * chunks + chunk) * kMaxProbes + p], summed on the host.
@@ -2224,274 +2170,6 @@ hipError_t launch_probe_dots(const ProbeSet &ps, const double *V, int64_t nslots
                        part);
     return hipGetLastError();
 }
-
-hipError_t launch_convolve(const double *x, const double *y, int64_t n, const double *grid, int64_t ng,
-                           double sigma, double *env, double *part, hipStream_t s) {
-    const int nb = (int)((ng + kBlock - 1) / kBlock);
-    hipLaunchKernelGGL(convolve_kernel, dim3(nb), dim3(kBlock), 0, s, x, y, n, grid, ng, sigma, env, part);
-    hipLaunchKernelGGL(convolve_norm_kernel, dim3(nb), dim3(kBlock), 0, s, env, ng, part, nb);
-    return hipGetLastError();
-}
-
-// ------------------------------------------------------------------------
-// Tridiagonal eigensolve (restates GIVENS, Source/yarkony.f90:91-543, for a
-// tridiagonal input: the Householder stage and the back transformation are
-// identities there).  The matrix arrives divided by its Frobenius norm.
-// ------------------------------------------------------------------------
-#define NV_EPS 1.1102230246251565e-16          /* 2^-53, determine_epsilon */
-#define NV_HUGE 1.7976931348623157e308
-#define NV_DEL1 (NV_EPS / 100.0)
-#define NV_DELTA (NV_EPS * NV_EPS * 100.0)
-#define NV_DELBIG (NV_HUGE * NV_DELTA / 1000.0)
-#define NV_THETA1 (1000.0 / NV_HUGE)
-#define NV_TOLER (NV_EPS * 100.0)
-
-// Number of eigenvalues below x: negative pivots of the LDL^T of T - x,
-// with a pivot below THETA1 in magnitude treated as in Source/yarkony.f90:360-389.
-__device__ int64_t sturm_below(const double *d, const double *e2, int64_t n, double x) {
-    int64_t nonneg = 0;
-    int64_t j = 0;
-    double f = d[0] - x;
-    while (true) {
-        if (fabs(f) < NV_THETA1) {
-            j += 2;
-            nonneg += 1;
-            if (j >= n) break;
-            f = d[j] - x;
-            continue;
-        }
-        if (f >= 0.0) nonneg += 1;
-        j += 1;
-        if (j >= n) break;
-        f = d[j] - x - e2[j - 1] / f;
-    }
-    return n - nonneg;
-}
-
-// One wave per root: multisection.  Each round the 64 lanes take Sturm counts
-// at 64 interior points of [lo, hi] and the wave keeps the sub-interval where
-// the count reaches i + 1 (count(lo) < i + 1 <= count(hi) throughout), so a
-// round shrinks the interval 65-fold where bisection halves it.  When the
-// points no longer fall strictly inside (a few ulps left) it bisects, and it
-// stops at adjacent doubles; the root is hi, as in the bisection of GIVENS
-// (Source/yarkony.f90:345-400).  T (d, e2) is staged in LDS when it fits
-// (lds = 1): every Sturm step reads it.
-constexpr int64_t kTriLdsMax = 4000;  // 2 * 4000 doubles, under 64 KB
-
-__global__ __launch_bounds__(64) void tri_bisect_kernel(int64_t n, const double *dg, const double *e2g,
-                                                         double *root, int lds) {
-    extern __shared__ double tri_lds[];
-    const double *d = dg, *e2 = e2g;
-    if (lds) {
-        for (int64_t k = threadIdx.x; k < n; k += blockDim.x) {
-            tri_lds[k] = dg[k];
-            tri_lds[n + k] = e2g[k];
-        }
-        __syncthreads();
-        d = tri_lds;
-        e2 = tri_lds + n;
-    }
-    const int64_t i = blockIdx.x;
-    const int lane = threadIdx.x;
-    double lo = -1.0, hi = 1.0;
-    for (int guard = 0; guard < 4096; ++guard) {
-        const double x = lo + (hi - lo) * ((double)(lane + 1) / 65.0);
-        const bool inside = x > lo && x < hi;
-        const bool ge = inside ? sturm_below(d, e2, n, x) >= i + 1 : x >= hi;
-        const unsigned long long ball = __ballot(ge);
-        const double xprev = __shfl_up(x, 1, 64);
-        const int k = ball ? __ffsll(ball) - 1 : 64;  // first point at or above the root
-        const double new_hi = k < 64 ? __shfl(x, k, 64) : hi;
-        const double new_lo = k == 0 ? lo : __shfl(k < 64 ? xprev : x, k < 64 ? k : 63, 64);
-        if ((new_lo > lo && new_lo < new_hi) || new_hi < hi) {
-            lo = new_lo > lo ? new_lo : lo;
-            hi = new_hi;
-            continue;
-        }
-        const double mid = (lo + hi) * 0.5;
-        if (mid == lo || mid == hi) break;
-        if (sturm_below(d, e2, n, mid) >= i + 1) hi = mid;
-        else lo = mid;
-    }
-    if (lane == 0) root[i] = hi;
-}
-
-// Back substitution through the pivoted factors of one root (Source/yarkony.f90:790-780).
-// Returns the last pivot used (the value the forward sweep of the reference
-// carries in TEMP).
-__device__ double tri_backsolve(int64_t n, int64_t i, const double *U2, const double *U3, const double *U4,
-                                double *v) {
-    double t = 1.0;
-    for (int64_t l = n - 1; l >= 0; --l) {
-        while (true) {
-            const double v1 = l + 1 < n ? v[(l + 1) * n + i] : 0.0;
-            const double v2 = l + 2 < n ? v[(l + 2) * n + i] : 0.0;
-            const double e = v[l * n + i] - v1 * U3[l * n + i] - v2 * U4[l * n + i];
-            // overflow guard of the reference; a non-finite value cannot be
-            // rescaled and ends the sweep instead of looping
-            if (fabs(e) > NV_DELBIG && isfinite(e)) {
-                for (int64_t k = 0; k < n; ++k) v[k * n + i] /= NV_DELBIG;
-                continue;
-            }
-            t = U2[l * n + i];
-            if (fabs(t) < NV_DELTA) t = NV_DELTA;
-            v[l * n + i] = e / t;
-            break;
-        }
-    }
-    return t;
-}
-
-// Inverse iteration for root i: factor T - root (partial pivoting), start
-// from ones (or the reference's multiplicative generator inside a cluster),
-// back solve, forward sweep, back solve.  Vectors are stored component-major:
-// vec[j*n + i].
-__global__ void tri_inverse_kernel(int64_t n, const double *d, const double *e, const double *root,
-                                   const int32_t *ia, const int64_t *rank, double *lu, double *vec) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int64_t nn = n * n;
-    double *U2 = lu, *U3 = lu + nn, *U4 = lu + 2 * nn, *U5 = lu + 3 * nn;
-    const double ar = root[i];
-    double el1 = d[0] - ar;
-    double el2 = n > 1 ? e[0] : 0.0;
-    for (int64_t j = 0; j + 1 < n; ++j) {
-        const double bj = e[j];
-        const double bj1 = j + 2 < n ? e[j + 1] : 0.0;
-        double t;
-        if (fabs(el1) <= fabs(bj)) {
-            U2[j * n + i] = bj;
-            U3[j * n + i] = d[j + 1] - ar;
-            U4[j * n + i] = bj1;
-            t = 1.0;
-            if (fabs(bj) > NV_THETA1) t = el1 / bj;
-            el1 = el2 - t * (d[j + 1] - ar);
-            el2 = -t * bj1;
-        } else {
-            U2[j * n + i] = el1;
-            U3[j * n + i] = el2;
-            U4[j * n + i] = 0.0;
-            t = bj / el1;
-            el1 = d[j + 1] - ar - t * el2;
-            el2 = bj1;
-        }
-        U5[j * n + i] = t;
-    }
-    U2[(n - 1) * n + i] = el1;
-    U3[(n - 1) * n + i] = 0.0;
-    U4[(n - 1) * n + i] = 0.0;
-    if (n >= 2) U4[(n - 2) * n + i] = 0.0;
-    // start vector
-    if (ia[i] == 0) {
-        for (int64_t j = 0; j < n; ++j) vec[j * n + i] = 1.0;
-    } else {
-        // state of x <- 4099 x mod 2^23 after n*rank[i] draws from 2^23-3
-        const uint64_t m = 1ull << 23;
-        uint64_t a = 4099, x = m - 3;
-        uint64_t k = (uint64_t)n * (uint64_t)rank[i];
-        uint64_t p = a % m, acc = 1;
-        while (k) {
-            if (k & 1) acc = (acc * p) % m;
-            p = (p * p) % m;
-            k >>= 1;
-        }
-        x = (x * acc) % m;
-        for (int64_t j = 0; j < n; ++j) {
-            x = (4099ull * x) % m;
-            vec[j * n + i] = (double)x / (double)(m / 2) - 1.0;
-        }
-    }
-    const double t1 = tri_backsolve(n, i, U2, U3, U4, vec);
-    // forward sweep (Source/yarkony.f90:890-830); a swapped row uses the last
-    // pivot of the back substitution as multiplier, as the reference does.
-    double el = vec[0 * n + i];
-    for (int64_t j = 0; j + 1 < n; ++j) {
-        const double nxt = vec[(j + 1) * n + i];
-        if (U2[j * n + i] == e[j]) {
-            vec[j * n + i] = nxt;
-            el = el - nxt * t1;
-        } else {
-            vec[j * n + i] = el;
-            el = nxt - el * U5[j * n + i];
-        }
-    }
-    vec[(n - 1) * n + i] = el;
-    tri_backsolve(n, i, U2, U3, U4, vec);
-}
-
-// Normalisation (Source/yarkony.f90:900-920) by one block: max |v|, sum of
-// (v/max)^2, scale, flush components below eps/100 to zero.
-__device__ void tri_normalize_block(int64_t n, int64_t i, double *vec) {
-    __shared__ double red[16];
-    double mx = 0.0;
-    for (int64_t j = threadIdx.x; j < n; j += blockDim.x) mx = fmax(fabs(vec[j * n + i]), mx);
-    for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off, 64));
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
-    __syncthreads();
-    mx = 0.0;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) mx = fmax(mx, red[w]);
-    double s = 0.0;
-    for (int64_t j = threadIdx.x; j < n; j += blockDim.x) {
-        const double q = vec[j * n + i] / mx;
-        s += q * q;
-    }
-    s = block_sum(s);
-    const double t = 1.0 / (sqrt(s) * mx);
-    for (int64_t j = threadIdx.x; j < n; j += blockDim.x) {
-        double v = vec[j * n + i] * t;
-        if (fabs(v) < NV_DEL1) v = 0.0;
-        vec[j * n + i] = v;
-    }
-    __syncthreads();
-}
-
-// Gram-Schmidt inside clusters of near-equal roots (Source/yarkony.f90:800-870)
-// and normalisation.  One block per root that starts a cluster (or stands
-// alone); the block walks the cluster's members in order.
-__global__ __launch_bounds__(256) void tri_finish_kernel(int64_t n, const int32_t *ia, double *vec) {
-    const int64_t i = blockIdx.x;
-    if (i >= n || ia[i] != 0) return;
-    tri_normalize_block(n, i, vec);
-    for (int64_t m = i + 1; m < n && ia[m] > 0; ++m) {
-        for (int64_t j1 = 1; j1 <= ia[m]; ++j1) {
-            const int64_t k = m - j1;
-            double t = 0.0;
-            for (int64_t j = threadIdx.x; j < n; j += blockDim.x) t += vec[j * n + m] * vec[j * n + k];
-            t = block_sum(t);
-            for (int64_t j = threadIdx.x; j < n; j += blockDim.x) vec[j * n + m] -= t * vec[j * n + k];
-            __syncthreads();
-        }
-        tri_normalize_block(n, m, vec);
-    }
-}
-
-__global__ void tri_cluster_kernel(int64_t n, const double *root, int32_t *ia, int64_t *rank) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    int32_t c = 0;
-    int64_t r = 0;
-    for (int64_t i = 0; i < n; ++i) {
-        if (i > 0 && fabs(root[i - 1] - root[i]) < NV_TOLER) c += 1;
-        else c = 0;
-        ia[i] = c;
-        rank[i] = r;
-        if (c != 0) r += 1;
-    }
-}
-
-hipError_t launch_tridiag(int64_t n, const TriWork &w, double anorm, hipStream_t s) {
-    (void)anorm;
-    const int tb = 64;
-    const int g = (int)((n + tb - 1) / tb);
-    const int lds = n <= kTriLdsMax;
-    hipLaunchKernelGGL(tri_bisect_kernel, dim3((unsigned)n), dim3(64), lds ? (size_t)2 * n * sizeof(double) : 0, s,
-                       n, w.d, w.e2, w.root, lds);
-    hipLaunchKernelGGL(tri_cluster_kernel, dim3(1), dim3(64), 0, s, n, w.root, w.ia, w.rank);
-    hipLaunchKernelGGL(tri_inverse_kernel, dim3(g), dim3(tb), 0, s, n, w.d, w.e, w.root, w.ia, w.rank, w.lu, w.vec);
-    hipLaunchKernelGGL(tri_finish_kernel, dim3((unsigned)n), dim3(256), 0, s, n, w.ia, w.vec);
-    return hipGetLastError();
-}
-
 
 // ------------------------------------------------------------------------
 // Batched Lanczos: many operators of uneven size advance one iteration per

@@ -107,8 +107,6 @@ hipError_t launch_finish_sum(const double *partials, int nparts, double *out, co
 hipError_t launch_norm_to(const double *v, int64_t n, double *out, double *partials, unsigned *counter,
                           hipStream_t s);
 
-// Normalised Gaussian envelope of sticks (x, y) on a grid; part holds
-// ceil(ng/256) doubles.
 // Dots of up to kMaxProbes probe vectors (length N) with the basis vectors
 // q_j0..q_{j0+nj-1} (slot j % nslots of V); part holds nj * probe_chunks(N) *
 // kMaxProbes partial sums, summed on the host per (j, probe).
@@ -120,21 +118,30 @@ struct ProbeSet {
 int probe_chunks(int64_t N);
 hipError_t launch_probe_dots(const ProbeSet &ps, const double *V, int64_t nslots, int64_t N, int64_t j0, int64_t nj,
                              double *part, hipStream_t s);
+// Normalised Gaussian envelope of sticks (x, y) on a grid; part holds
+// convolve_parts(ng) doubles (nv_spectrum.hip).
+int64_t convolve_parts(int64_t ng);
 hipError_t launch_convolve(const double *x, const double *y, int64_t n, const double *grid, int64_t ng,
                            double sigma, double *env, double *part, hipStream_t s);
 
-// ---- tridiagonal eigensolve ----
+// ---- tridiagonal eigensolve (nv_tridiag.hip) ----
+constexpr int kTriPad = 16;  // rows of TriWork::de past the matrix that a prefetch may read
 struct TriWork {
+    double *de = nullptr;    // [n + kTriPad][2]: normalised diagonal d_j, e_{j-1}^2 (rows past n zero)
     double *d = nullptr;     // [n] normalised diagonal
     double *e = nullptr;     // [n] normalised off-diagonal, e[j] couples j, j+1
-    double *e2 = nullptr;    // [n] squares
     double *root = nullptr;  // [n]
     double *vec = nullptr;   // [n][n], vec[j*n + i] = component j of root i
-    double *lu = nullptr;    // [5][n][n] per-root elimination rows, interleaved by root
+    double *lu = nullptr;    // [4][n][n] per-root elimination rows, interleaved by root
+    int32_t *cnt = nullptr;  // [tri_grid_points(n)] Sturm counts of a uniform grid
     int32_t *ia = nullptr;   // [n] position inside a cluster of near-equal roots
     int64_t *rank = nullptr; // [n] number of cluster members (ia>0) before root i
 };
-hipError_t launch_tridiag(int64_t n, const TriWork &w, double anorm, hipStream_t s);
+// Smallest e^2 in TriWork::de (the host applies it): a zero one would stop the product form of the
+// Sturm sequence at an exactly zero pivot.
+constexpr double kTriMinE2 = 1e-200;
+int tri_grid_points(int64_t n);
+hipError_t launch_tridiag(int64_t n, const TriWork &w, hipStream_t s);
 
 // ---- Ritz vectors and root analysis (nv_roots.hip) ----
 constexpr int kRitzChunk = 16;  // Ritz vectors formed per pass over the basis
