@@ -6,6 +6,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <map>
 #include <mutex>
 #include <string>
@@ -1357,6 +1358,101 @@ static int32_t ensure_gop(nv_ctx *c) {
     return NV_OK;
 }
 
+// The device side of the parameter derivatives: the forms of every monomial,
+// accumulated over pairs of vectors, by nv::launch_bilinear where it applies and
+// term by term otherwise.
+struct GradSums {
+    bool tiles = false;      // launch_bilinear
+    nv::GradModes modes{};
+    double *part = nullptr, *acc = nullptr;
+    size_t acc_count = 0;
+};
+
+// Allocates them for up to `pairs` pairs per call (through alloc) and clears the sums.
+static hipError_t grad_begin(nv_ctx *c, GradSums &gs, int pairs,
+                             const std::function<hipError_t(size_t, void **)> &alloc) {
+    const nv::Operator &op = c->op;
+    const int ns = (int)op.ns, M = (int)op.M, nss = ns * ns;
+    gs.tiles = nv::bilinear_ok(ns, M, (int)op.ordr);
+    size_t part;
+    if (gs.tiles) {
+        gs.modes.M = M;
+        gs.modes.D = (int32_t)op.D;
+        for (int k = 0; k < M; ++k) {
+            gs.modes.nf[k] = (int32_t)op.nfunc[k];
+            gs.modes.shft[k] = (int32_t)op.shft[k];
+            gs.modes.inv[k] = 1.0 / (double)op.nfunc[k];
+        }
+        part = nv::bilinear_part_bytes(ns, M, op.D, pairs);
+        gs.acc_count = (size_t)nv::bilinear_tiles(ns, M) * 256;
+    } else {
+        const int groups = nv::grad_groups(c->gdev);
+        part = (size_t)groups * nv::grad_chunks(c->gdev) * nss * 8;
+        gs.acc_count = (size_t)groups * nss;
+    }
+    hipError_t e = alloc(part, (void **)&gs.part);
+    if (e == hipSuccess) e = alloc(gs.acc_count * 8, (void **)&gs.acc);
+    if (e == hipSuccess) e = hipMemsetAsync(gs.acc, 0, gs.acc_count * 8, c->stream);
+    return e;
+}
+
+// Adds the forms of m <= pairs pairs: u_j at u + j*N, v_j in slot (slot0 + j) % nslots of v.
+static hipError_t grad_add(nv_ctx *c, const GradSums &gs, const double *u, const double *v, int64_t slot0,
+                           int64_t nslots, int m) {
+    const int64_t N = c->op.N;
+    if (gs.tiles)
+        return nv::launch_bilinear(gs.modes, (int)c->op.ns, u, N, v, N, slot0, nslots, m, gs.part, gs.acc, c->stream);
+    hipError_t e = hipSuccess;
+    for (int j = 0; j < m && e == hipSuccess; ++j)
+        e = nv::launch_grad_contract(c->gdev, u + j * N, v + ((slot0 + j) % nslots) * N, gs.part, gs.acc, c->stream);
+    return e;
+}
+
+// The sums in the order map_gradients reads them (the groups of grad_contract).
+static hipError_t grad_end(nv_ctx *c, const GradSums &gs, std::vector<double> &gh) {
+    std::vector<double> h(gs.acc_count);
+    hipError_t e = hipMemcpyAsync(h.data(), gs.acc, h.size() * 8, hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    if (e != hipSuccess) return e;
+    if (!gs.tiles) {
+        gh.swap(h);
+        return hipSuccess;
+    }
+    const nv::Operator &g = c->gop;
+    const int ns = (int)g.ns, M = (int)g.M, nss = ns * ns, nT = c->gdev.nterms, nD = c->gdev.ndterms;
+    gh.assign((size_t)nv::grad_groups(c->gdev) * nss, 0.0);
+    auto uv = [&](int k, int a, int l, int b) { return h[nv::bilinear_index(ns, M, k, a, l, b)]; };
+    auto wt = [&](int w, int a, int b) { return h[nv::bilinear_weight_index(ns, M, w, a, b)]; };
+    for (int a = 0; a < ns; ++a)
+        for (int b = 0; b < ns; ++b) {
+            const int ab = a * ns + b;
+            for (size_t t = 0; t < g.terms.size(); ++t) {
+                const nv::Term &tm = g.terms[t];
+                const int dt = g.term_dev[t], dd = g.term_ddev[t];
+                const int k = tm.mode[0];
+                double off, dia = 0.0;
+                if (tm.cnt == 2) {
+                    const int l = tm.mode[1];
+                    off = uv(std::min(k, l) + 1, a, std::max(k, l) + 1, b);
+                } else if (tm.pow[0] == 1) {
+                    off = uv(0, a, k + 1, b);
+                } else {
+                    dia = wt(k, a, b);
+                    off = uv(k + 1, a, k + 1, b) - (dia - wt(M + k, a, b));
+                }
+                if (dt >= 0) gh[(size_t)dt * nss + ab] = off;
+                if (dd >= 0) gh[(size_t)(nT + dd) * nss + ab] = dia;
+            }
+            gh[(size_t)(nT + nD + M) * nss + ab] = wt(2 * M, a, b);
+        }
+    for (int k = 0; k < M; ++k) {
+        double s = 0.0;
+        for (int a = 0; a < ns; ++a) s += wt(k, a, a);
+        gh[(size_t)(nT + nD + k) * nss] = s;
+    }
+    return hipSuccess;
+}
+
 // Maps the accumulated bilinear forms onto the nadvibs.in slots and the
 // frequencies (chain rule through c * prod_k w_k^{-p_k/2}, Source/top.f90:212-217).
 static void map_gradients(nv_ctx *c, const std::vector<double> &gacc, double *g_omega, double *g_concoef,
@@ -1472,8 +1568,6 @@ int32_t nv_lanczos_adjoint(nv_ctx *c, int64_t n, const double *abar, const doubl
     if (rc != NV_OK) return rc;
     const int64_t N = c->op.N, niter = c->opts.niter;
     const int64_t K = archive ? n : c->opts.checkpoint;
-    const int nss = (int)(c->op.ns * c->op.ns);
-    const int groups = nv::grad_groups(c->gdev), chunks = nv::grad_chunks(c->gdev);
     std::vector<double> beta_h(niter + 3);
     NV_HIP(c, hipMemcpy(beta_h.data(), c->st.beta, (niter + 3) * sizeof(double), hipMemcpyDeviceToHost));
     std::vector<void *> tmp;
@@ -1482,19 +1576,19 @@ int32_t nv_lanczos_adjoint(nv_ctx *c, int64_t n, const double *abar, const doubl
         if (er == hipSuccess) tmp.push_back(*p);
         return er;
     };
-    double *qb[3], *ub = nullptr, *hub = nullptr, *part = nullptr, *gpart = nullptr, *scal = nullptr;
-    double *abar_d = nullptr, *bbar_d = nullptr, *gacc = nullptr, *seg = nullptr, *ta = nullptr, *tb = nullptr;
+    double *qb[3], *ub = nullptr, *hub = nullptr, *part = nullptr, *scal = nullptr;
+    double *abar_d = nullptr, *bbar_d = nullptr, *seg = nullptr, *ta = nullptr, *tb = nullptr;
+    GradSums gs;
     hipError_t e = alloc((size_t)3 * N * 8, (void **)&qb[0]);
     qb[1] = qb[0] + N;
     qb[2] = qb[0] + 2 * N;
     if (e == hipSuccess) e = alloc((size_t)N * 8, (void **)&ub);
     if (e == hipSuccess) e = alloc((size_t)N * 8, (void **)&hub);
     if (e == hipSuccess) e = alloc((size_t)5 * nv::adj_blocks(N) * 8, (void **)&part);
-    if (e == hipSuccess) e = alloc((size_t)groups * chunks * nss * 8, (void **)&gpart);
     if (e == hipSuccess) e = alloc(8 * 8, (void **)&scal);
     if (e == hipSuccess) e = alloc((size_t)(n + 1) * 8, (void **)&abar_d);
     if (e == hipSuccess) e = alloc((size_t)(n + 2) * 8, (void **)&bbar_d);
-    if (e == hipSuccess) e = alloc((size_t)groups * nss * 8, (void **)&gacc);
+    if (e == hipSuccess) e = grad_begin(c, gs, 1, alloc);
     if (!archive) {
         if (e == hipSuccess) e = alloc((size_t)(K + 2) * N * 8, (void **)&seg);
         if (e == hipSuccess) e = alloc((size_t)(niter + 3) * 8, (void **)&ta);
@@ -1509,7 +1603,6 @@ int32_t nv_lanczos_adjoint(nv_ctx *c, int64_t n, const double *abar, const doubl
     e = hipMemcpyAsync(abar_d, abar, n * 8, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = hipMemcpyAsync(bbar_d, bbar, (n + 1) * 8, hipMemcpyHostToDevice, s);
     if (e == hipSuccess) e = hipMemsetAsync(qb[0], 0, (size_t)3 * N * 8, s);
-    if (e == hipSuccess) e = hipMemsetAsync(gacc, 0, (size_t)groups * nss * 8, s);
     int ia = 0, ib = 1, ic = 2;  // qbar_{i+1}, qbar_i, qbar_{i-1}
     bool have_hub = false;
     const int64_t nseg = (n + K - 1) / K;
@@ -1533,16 +1626,15 @@ int32_t nv_lanczos_adjoint(nv_ctx *c, int64_t n, const double *abar, const doubl
                                     abar_d, bbar_d, part, scal, ub, qb[ib], qb[ic], s);
             if (e == hipSuccess) e = hv_apply(c, prec, ub, hub, s);
             if (e == hipSuccess && c->dev.offstate) e = nv::launch_adj_transpose(c->dev, ub, hub, s);
-            if (e == hipSuccess) e = nv::launch_grad_contract(c->gdev, ub, qi, gpart, gacc, s);
+            if (e == hipSuccess) e = grad_add(c, gs, ub, qi, 0, 1, 1);
             if (e == hipSuccess) e = nv::launch_adj_zero(N, qb[ia], s);
             have_hub = true;
             const int t = ia;
             ia = ib; ib = ic; ic = t;
         }
     }
-    std::vector<double> gh((size_t)groups * nss);
-    if (e == hipSuccess) e = hipMemcpyAsync(gh.data(), gacc, gh.size() * 8, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    std::vector<double> gh;
+    if (e == hipSuccess) e = grad_end(c, gs, gh);
     if (e != hipSuccess) return done(hip_fail(c, e, "adjoint"));
     map_gradients(c, gh, g_omega, g_concoef, g_potterms);
     return done(NV_OK);
@@ -1626,9 +1718,7 @@ int32_t nv_krylov_gradient(nv_ctx *c, int64_t n, const double *tbar, double *g_o
     if (rc != NV_OK) return rc;
     const int64_t N = c->op.N, niter = c->opts.niter;
     const int64_t K = archive ? n : c->opts.checkpoint;
-    const int nss = (int)(c->op.ns * c->op.ns);
-    const int groups = nv::grad_groups(c->gdev), chunks = nv::grad_chunks(c->gdev);
-    const int64_t jc = std::min<int64_t>(K, 4 * nv::kRitzChunk);
+    const int64_t jc = std::min<int64_t>(K, nv::kRitzChunk);
     std::vector<void *> tmp;
     auto alloc = [&](size_t bytes, void **p) -> hipError_t {
         hipError_t er = hipMalloc(p, bytes);
@@ -1639,12 +1729,12 @@ int32_t nv_krylov_gradient(nv_ctx *c, int64_t n, const double *tbar, double *g_o
         for (void *p : tmp) hipFree(p);
         return code;
     };
-    double *tb = nullptr, *W = nullptr, *gpart = nullptr, *gacc = nullptr;
+    double *tb = nullptr, *W = nullptr;
+    GradSums gs;
     double *segA = nullptr, *segB = nullptr, *ta = nullptr, *tbb = nullptr;
     hipError_t e = alloc((size_t)n * n * 8, (void **)&tb);
     if (e == hipSuccess) e = alloc((size_t)jc * N * 8, (void **)&W);
-    if (e == hipSuccess) e = alloc((size_t)groups * chunks * nss * 8, (void **)&gpart);
-    if (e == hipSuccess) e = alloc((size_t)groups * nss * 8, (void **)&gacc);
+    if (e == hipSuccess) e = grad_begin(c, gs, (int)jc, alloc);
     if (!archive) {
         if (e == hipSuccess) e = alloc((size_t)2 * (K + 2) * N * 8, (void **)&segA);
         segB = segA + (K + 2) * N;
@@ -1654,7 +1744,6 @@ int32_t nv_krylov_gradient(nv_ctx *c, int64_t n, const double *tbar, double *g_o
     if (e != hipSuccess) return done(hip_fail(c, e, "krylov gradient allocation"));
     hipStream_t s = c->stream;
     e = hipMemcpyAsync(tb, tbar, (size_t)n * n * 8, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = hipMemsetAsync(gacc, 0, (size_t)groups * nss * 8, s);
     // Sum over j in [o0, o1] of q_j^T (dH/dtheta) w_j, w_j = sum_{k=i0..i1} Tbar[j][k] q_k: q_j in
     // slot (j % ons) of obuf, q_k in slot (k % ins) of ibuf.  Tbar is symmetric, so its rows
     // serve as the component-major coefficient table of launch_ritz_vectors.
@@ -1664,8 +1753,7 @@ int32_t nv_krylov_gradient(nv_ctx *c, int64_t n, const double *tbar, double *g_o
             const int64_t m = std::min(jc, o1 - j0 + 1);
             e = nv::launch_ritz_vectors(ibuf, N, i1 - i0 + 1, tb + (i0 - 1) * n + (j0 - 1), n, m, i0 % ins, ins, W,
                                         s);
-            for (int64_t j = 0; j < m && e == hipSuccess; ++j)
-                e = nv::launch_grad_contract(c->gdev, W + j * N, obuf + ((j0 + j) % ons) * N, gpart, gacc, s);
+            if (e == hipSuccess) e = grad_add(c, gs, W, obuf, j0 % ons, ons, (int)m);
         }
     };
     // Orthogonality of the basis the projection assumes: probe vectors against every later
@@ -1731,9 +1819,8 @@ int32_t nv_krylov_gradient(nv_ctx *c, int64_t n, const double *tbar, double *g_o
             }
         }
     }
-    std::vector<double> gh((size_t)groups * nss);
-    if (e == hipSuccess) e = hipMemcpyAsync(gh.data(), gacc, gh.size() * 8, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    std::vector<double> gh;
+    if (e == hipSuccess) e = grad_end(c, gs, gh);
     if (e != hipSuccess) return done(hip_fail(c, e, "krylov gradient"));
     map_gradients(c, gh, g_omega, g_concoef, g_potterms);
     if (worst > 1e-4) {

@@ -143,8 +143,8 @@ constexpr double kTriMinE2 = 1e-200;
 int tri_grid_points(int64_t n);
 hipError_t launch_tridiag(int64_t n, const TriWork &w, hipStream_t s);
 
-// ---- Ritz vectors and root analysis (nv_roots.hip) ----
-constexpr int kRitzChunk = 16;  // Ritz vectors formed per pass over the basis
+// ---- Ritz vectors (nv_contract.hip) and root analysis (nv_roots.hip) ----
+constexpr int kRitzChunk = 64;  // Ritz vectors formed per pass over the basis
 constexpr int kRitzKB = 64;     // basis vectors per LDS stage of the eigenvectors
 constexpr int kGramT = 32;      // Gram tile edge
 // Y[i][r] = sum_k vec[k*n + i] V[k*N + r], i < nroots, k < n.
@@ -220,6 +220,23 @@ int grad_chunks(const NvOpDev &g);
 size_t grad_lds_bytes(const NvOpDev &g);
 hipError_t launch_grad_contract(const NvOpDev &g, const double *ub, const double *q, double *part, double *gacc,
                                 hipStream_t s);
+// The same forms for expansions up to second order, of m pairs of vectors in one launch
+// (nv_contract.hip): u at u + j*ldu, v at v + ((slot0 + j) % nslots)*ldv, j = 0..m-1, added to acc.
+struct GradModes {
+    int32_t M, D;
+    int32_t nf[16], shft[16];
+    double inv[16];  // 1 / nf
+};
+bool bilinear_ok(int ns, int M, int ordr);
+int bilinear_tiles(int ns, int M);  // acc holds bilinear_tiles * 256 doubles
+size_t bilinear_part_bytes(int ns, int M, int64_t D, int m);
+// Where acc holds (q_k u_a) . (q_l v_c), k <= l (0: the vector itself, 1..M: modes), and
+// sum_r w u_a v_c for weight w: n_k + 1/2 (w = k), the last function of mode k at nf_k/2
+// (w = M + k), 1 (w = 2M); modes counted from 0 there.
+int bilinear_index(int ns, int M, int k, int a, int l, int c);
+int bilinear_weight_index(int ns, int M, int w, int a, int c);
+hipError_t launch_bilinear(const GradModes &g, int ns, const double *u, int64_t ldu, const double *v, int64_t ldv,
+                           int64_t slot0, int64_t nslots, int m, double *part, double *acc, hipStream_t s);
 // Broadened spectrum of tridiagonal eigenpairs (theta on the device, vec as
 // TriWork::vec) and its adjoint; work holds 2n + 8 + 2n^2 doubles.
 hipError_t launch_spec_env(int64_t n, const double *theta, const double *vec, double ref, double c, double sigma,
