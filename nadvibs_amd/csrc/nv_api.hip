@@ -56,6 +56,7 @@ struct nv_ctx {
     nv::JitKernels jit[2];
     std::string jit_log;
     float *hx32 = nullptr;
+    void *yt[2] = {nullptr, nullptr};     // slab pass of a standalone fast-block H*v, FP64 and FP32 (in allocs)
     double *hx64i = nullptr;              // interleaved FP64 copy of a standalone H*v input (two-pass form)
     void *z2 = nullptr;                   // channel scratch of the two-pass H*v
     size_t z2_bytes = 0;
@@ -306,6 +307,24 @@ int32_t nv_create(const nv_problem *prob, int32_t device, nv_ctx **out) {
                 }
             }
             std::vector<float> t32(op.fb_tab.begin(), op.fb_tab.end());
+            // the coupling matrices in the order the sweep reads them
+            std::vector<double> fc;
+            for (int ph = 0; ph < 3; ++ph) {
+                f.cbase[ph] = (int32_t)fc.size();
+                const int c0 = ph == 0 ? 4 : 0, c1 = ph == 0 ? NV_FB_NCH : ph == 1 ? 4 : 1;
+                const int t0 = op.fb_sgrp[ph == 2 ? 2 : 0][0], t1 = op.fb_sgrp[ph][NV_FB_NSLOW];
+                for (int t = t0; t < t1; ++t)
+                    for (int q = c0; q < c1; ++q) {
+                        const int m = op.fb_S[t].cm[q];
+                        for (int64_t a = 0; a < op.ns; ++a)
+                            for (int64_t b = 0; b <= a; ++b)
+                                fc.push_back(m >= 0 ? op.cmat[((size_t)m * op.ns + a) * op.ns + b] : 0.0);
+                    }
+            }
+            if (fc.empty()) fc.push_back(0.0);
+            std::vector<float> fc32(fc.begin(), fc.end());
+            if (e == hipSuccess) e = upload(c, fc, &f.c64, c->allocs);
+            if (e == hipSuccess) e = upload(c, fc32, &f.c32, c->allocs);
             if (e == hipSuccess) e = upload(c, op.fb_S, &f.S, c->allocs);
             if (e == hipSuccess) e = upload(c, op.fb_steps, &f.steps, c->allocs);
             if (e == hipSuccess && !op.fb_pure.empty()) e = upload(c, op.fb_pure, &f.pure, c->allocs);
@@ -314,6 +333,56 @@ int32_t nv_create(const nv_problem *prob, int32_t device, nv_ctx **out) {
             if (e == hipSuccess) e = upload(c, t32, &f.tab32, c->allocs);
             f.on = e == hipSuccess ? 1 : 0;
         }
+    }
+    d.slab = NvSlabDev{};
+    // A slab pass of its own from 200 steps of degree three over the slow modes (five or more modes
+    // of a cubic operator): 88.5M elements, 560 steps, 10.6 -> 8.0 ms (FP32) and 23.0 -> 17.4 ms
+    // (FP64); two states, 3.6M rows, 220 steps: 1,091 -> 911 us and 1,125 -> 1,117 us; with 120 or 56
+    // the extra pass over the vectors costs what the steps do (three states, 1.3M rows, FP64: 406
+    // against 441 us; four, 1.4M rows: 361 against 426 us).  NV_HV_FB=1 takes it always.
+    if (d.fb.on && op.slab && (op.slab_steps >= 200 || d.fb_min_bytes == 0)) {
+        NvSlabDev &l = d.slab;
+        l.gl = op.slab_gl;
+        l.nl = op.slab_nl;
+        l.gpts = op.slab_gpts;
+        l.pts = op.slab_pts;
+        for (int k = 0; k < NV_SLAB_NL; ++k) {
+            l.lnf[k] = k < op.slab_nl ? (int32_t)op.nfunc[op.slab_gl + k] : 1;
+            l.c3[k] = op.slab_c3[k];
+        }
+        for (int k = 0; k < 6; ++k) l.c21[k] = op.slab_c21[k];
+        l.c111 = op.slab_c111;
+        l.r64 = op.slab_r64;
+        l.r32 = op.slab_r32;
+        l.R64 = op.slab_R64;
+        l.R32 = op.slab_R32;
+        for (int q = 0; q < NV_FB_NSLOW; ++q) l.s2end[q] = op.slab_s2end[q];
+        l.kl = op.slab_kl;
+        l.kpts = op.slab_kpts;
+        l.kr64 = op.slab_kr64;
+        l.kr32 = op.slab_kr32;
+        for (int k = 0; k < NV_LEAD_NL; ++k) {
+            l.knf[k] = k < op.slab_kl ? (int32_t)op.nfunc[k] : 1;
+            l.k3[k] = op.slab_k3[k];
+            l.k111[k] = op.slab_k111[k];
+        }
+        for (int k = 0; k < NV_LEAD_NL * (NV_LEAD_NL - 1); ++k) l.k21[k] = op.slab_k21[k];
+        std::vector<float> k32(op.slab_ktab.begin(), op.slab_ktab.end());
+        if (e == hipSuccess) e = upload(c, op.slab_ktab, &l.ktab64, c->allocs);
+        if (e == hipSuccess) e = upload(c, k32, &l.ktab32, c->allocs);
+        for (int q = 0; q < 4; ++q) l.ggrp[q] = op.slab_ggrp[q];
+        for (int q = 0; q <= NV_FB_NSLOW; ++q) l.sgrp[q] = op.slab_sgrp[q];
+        l.ntab = (int32_t)(op.slab_tabdiv.size() / 2);
+        std::vector<float> t32(op.slab_tab.begin(), op.slab_tab.end()), l32(op.slab_ltab.begin(), op.slab_ltab.end());
+        if (e == hipSuccess) e = upload(c, op.slab_G, &l.G, c->allocs);
+        if (e == hipSuccess) e = upload(c, op.slab_S, &l.S, c->allocs);
+        if (e == hipSuccess) e = upload(c, op.slab_tabdiv, &l.tabdiv, c->allocs);
+        if (e == hipSuccess) e = upload(c, op.slab_tab, &l.tab64, c->allocs);
+        if (e == hipSuccess) e = upload(c, t32, &l.tab32, c->allocs);
+        if (e == hipSuccess) e = upload(c, op.slab_ltab, &l.ltab64, c->allocs);
+        if (e == hipSuccess) e = upload(c, l32, &l.ltab32, c->allocs);
+        l.on = e == hipSuccess ? 1 : 0;
+        if (e == hipSuccess) e = nv::hv_slab_prepare(d);
     }
     {
         const char *k = std::getenv("NV_HV_KERNEL");
@@ -515,13 +584,29 @@ static hipError_t interleaved_input(nv_ctx *c, int32_t prec, const double *x, co
     return e;
 }
 
+// The slab pass's buffer for precision prec, or null when the operator has no
+// slab pass or the memory is short (the sweep then takes every step itself).
+static void *alloc_slab(nv_ctx *c, int32_t prec, std::vector<void *> &owner) {
+    const size_t bytes = nv::hv_slab_bytes(c->dev, prec);
+    void *p = nullptr;
+    if (bytes == 0) return nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    owner.push_back(p);
+    return p;
+}
+
 // y = H x (double in and out) on stream s, couplings in precision prec.
 static hipError_t hv_apply(nv_ctx *c, int32_t prec, const double *x, double *y, hipStream_t s) {
     if (use_fb(c, prec)) {
         const void *xin = nullptr;
         hipError_t e = interleaved_input(c, prec, x, &xin, s);
         if (e != hipSuccess) return e;
-        return nv::launch_hv_fb_full(c->dev, prec, x, xin, y, s);
+        void *&yt = c->yt[prec == NV_PREC_F32];
+        if (!yt) yt = alloc_slab(c, prec, c->allocs);
+        return nv::launch_hv_fb_full(c->dev, prec, x, xin, yt, y, s);
     }
     if (use_hv2(c, prec)) {
         hipError_t e = ensure_z2(c, nv::hv2_scratch_bytes(c->dev, prec));
@@ -727,6 +812,8 @@ int32_t nv_lanczos_init(nv_ctx *c, const nv_lanczos_opts *o) {
         NV_HIP(c, ensure_z2(c, nv::hv2_scratch_bytes(c->dev, o->prec)));
         st.z2 = c->z2;
     }
+    // (last, after what the run cannot do without)
+    if (!st.yt && !jit && use_fb(c, o->prec)) st.yt = alloc_slab(c, o->prec, c->lz_allocs);
     // start vector in the slot of iteration 1, beta(0) = |start|
     double *s1 = st.V + (1 % st.nslots) * N;
     int32_t rc = build_start(c, s1);

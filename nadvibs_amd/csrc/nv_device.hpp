@@ -123,6 +123,7 @@ struct NvFbS {
     int32_t nd;            // slow slots whose only step is Delta = 0 (at most 2)
     int32_t dtab[2];       // their factor rows; entry 0 is h(p, n, 0)
     int32_t cm[NV_FB_NCH]; // per channel: coupling matrix (row of cmat) of the term (S, F), or -1
+    int32_t cmask;         // channels c with cm[c] >= 0
     int32_t excl0;         // channel 0 leaves out the middle step Delta_s = 0 (all stepping slots even)
     int32_t nchk;          // 1 + the last channel c with cm[c] >= 0 (channels are ordered by the
                            // degree of their fast monomial)
@@ -150,11 +151,62 @@ struct NvFbDev {
     const float *tab32;
     const NvFbS *S;        // grouped by phase, then by slow shape
     int32_t sgrp[3][NV_FB_NSLOW + 1];  // phase 0: nchk > 4, phase 1: 1 < nchk <= 4, phase 2: nchk == 1
+    const double *c64;     // coupling matrices (lower triangles, zero where cm[c] < 0) in the order of S: from
+    const float *c32;      //   cbase[0] channels 4.. of phase 0's monomials, from cbase[1] channels 0..3 of phase
+    int32_t cbase[3];      //   0's and 1's, from cbase[2] channel 0 of phase 2's
     int32_t nch;           // channels in use
     int32_t chs[NV_FB_NCH + 1];  // fast steps of channel c: [chs[c], chs[c+1]) (c >= 1)
     const NvStep *steps;   // fast steps: stride = lane offset; factors (mode, ftab row)
     int32_t npure;
     const NvFbPure *pure;
+};
+
+// Slab H*v: the terms of degree three over the slow modes alone, taken out of
+// the fast-block sweep (they hold most of its loads: 560 of the 680 of a cubic
+// operator on seven slow modes).  The slow modes split into G = 0..gl-1 and
+// L = gl..mf-1; a workgroup owns every point of the L modes times r
+// consecutive fast rows for one set of G digits, one or two rows of a point per
+// thread.
+// A monomial is a product S_G S_L: each distinct S_G of degree < 3 is gathered
+// once, u = S_G x, published in LDS, and every S_L it pairs with is read from
+// there; S_L = 1 adds u itself.
+// The terms of degree three within the leading kl modes alone (most of the
+// S_G of degree three) are a pass of their own: a workgroup holds a few rows of
+// every point of those modes in LDS, reads each once and needs no gather.
+#define NV_SLAB_NL 3
+#define NV_LEAD_NL 4
+#define NV_LEAD_LDS (152 * 1024)  // of the 160 KB of a CU
+struct NvSlabG {           // S_G of degree 1 or 2
+    int32_t base, inc[3], tab[3];  // steps as in NvFbS, p + 1 slots for power p
+    int32_t c1[NV_SLAB_NL];        // degree 2: cmat row of the term with S_L = q_k, or -1
+    int32_t c2[NV_SLAB_NL];        // degree 1: q_k^2
+    int32_t c11[3];                // degree 1: q_0 q_1, q_0 q_2, q_1 q_2
+};
+struct NvSlabDev {
+    int32_t on;
+    int32_t gl, nl;        // first L mode, L modes (1..NV_SLAB_NL)
+    int32_t gpts, pts;     // points of the G and of the L modes
+    int32_t lnf[NV_SLAB_NL];
+    int32_t r64, r32;      // fast rows per workgroup (divisors of the fast block's P)
+    int32_t R64, R32;      // of which a thread takes 1 or 2
+    int32_t s2end[NV_FB_NSLOW];     // the fast-block sweep's phase 2 stops here in each shape group (monomials of
+                                    // degree three have fewer steps, other shapes, on modes of few functions)
+    int32_t ggrp[4];       // S_G of shapes (2), (3), (2,2)
+    int32_t sgrp[NV_FB_NSLOW + 1];  // S_G of degree 3, by slow shape
+    int32_t c3[NV_SLAB_NL], c21[6], c111;  // S_G = 1: q_k^3, q_k^2 q_l (k * 2 + (l < k ? l : l - 1)), q_0 q_1 q_2
+    // the leading pass (kl = 0: none): its modes, points, rows per workgroup, terms and factors
+    int32_t kl, kpts, kr64, kr32, knf[NV_LEAD_NL];
+    int32_t k3[NV_LEAD_NL], k21[NV_LEAD_NL * (NV_LEAD_NL - 1)], k111[4];  // (0,1,2) (0,1,3) (0,2,3) (1,2,3)
+    const double *ktab64;  // [kl][nmax][9] as ltab
+    const float *ktab32;
+    int32_t ntab;
+    const int32_t *tabdiv; // [ntab][2]: a factor row's mode digit is (g / [0]) % [1]
+    const NvSlabG *G;
+    const NvFbS *S;
+    const double *tab64;   // [ntab][nmax][4]: h(p, n, -p + 2i), 0 outside the basis
+    const float *tab32;
+    const double *ltab64;  // [nl][nmax][9]: h(1, n, -1..1), h(2, n, -2..2), h(3, n, -3..3)
+    const float *ltab32;
 };
 
 // Everything the H*v kernels read, passed by value.
@@ -180,6 +232,7 @@ struct NvOpDev {
     int64_t hv2_min_bytes;          // vector size from which the two-pass H*v serves the iteration
     NvFbDev fb;                     // fast-block H*v tables (fb.on = 0: not available)
     int64_t fb_min_bytes;           // vector size from which the fast-block H*v serves
+    NvSlabDev slab;                 // its degree-three slow terms as a pass of their own (slab.on = 0: none)
     int32_t stream_nt;              // vectors far beyond the caches: the step, the normalisation and
                                     // the fast-block H*v's epilogue stream them with non-temporal accesses
 };

@@ -12,133 +12,10 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <hip/hip_bf16.h>
 
-#include <type_traits>
-
-#include "nv_kernels.hpp"
+#include "nv_hvcore.hpp"
 
 namespace nv {
-
-// Workgroups of one launch go to the 8 XCDs round-robin (workgroup b to XCD
-// b % 8).  H*v gathers x at +-stride of every mode, so a workgroup reads the
-// rows of its neighbours along the slow modes; mapping each XCD onto one
-// contiguous range of rows keeps that window inside the XCD's own L2.
-__device__ __forceinline__ int xcd_block(int b, int g) {
-    const int x = b & 7, j = b >> 3, q = g >> 3, rem = g & 7;
-    return x * q + (x < rem ? x : rem) + j;
-}
-
-// ------------------------------------------------------------------------
-// reductions
-// ------------------------------------------------------------------------
-__device__ __forceinline__ double wave_sum(double v) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
-// Block-wide sum; every thread gets the result.  blockDim.x <= 1024.
-__device__ double block_sum(double v) {
-    __shared__ double red[16];
-    v = wave_sum(v);
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    __syncthreads();
-    if (lane == 0) red[wid] = v;
-    __syncthreads();
-    const int nw = (blockDim.x + 63) >> 6;
-    double t = 0.0;
-    for (int i = 0; i < nw; ++i) t += red[i];
-    return t;
-}
-
-// ------------------------------------------------------------------------
-// element types
-// ------------------------------------------------------------------------
-template <typename T> __device__ __forceinline__ float to_f(T v);
-template <> __device__ __forceinline__ float to_f<float>(float v) { return v; }
-template <> __device__ __forceinline__ float to_f<__hip_bfloat16>(__hip_bfloat16 v) { return __bfloat162float(v); }
-
-template <typename TIn, typename TAcc> __device__ __forceinline__ TAcc load_acc(const TIn *p);
-template <> __device__ __forceinline__ double load_acc<double, double>(const double *p) { return *p; }
-template <> __device__ __forceinline__ float load_acc<float, float>(const float *p) { return *p; }
-template <> __device__ __forceinline__ float load_acc<__hip_bfloat16, float>(const __hip_bfloat16 *p) {
-    return __bfloat162float(*p);
-}
-template <> __device__ __forceinline__ float load_acc<double, float>(const double *p) { return (float)*p; }
-
-template <typename T> __device__ __forceinline__ T from_d(double v);
-template <> __device__ __forceinline__ double from_d<double>(double v) { return v; }
-template <> __device__ __forceinline__ float from_d<float>(double v) { return (float)v; }
-template <> __device__ __forceinline__ __hip_bfloat16 from_d<__hip_bfloat16>(double v) {
-    return __float2bfloat16((float)v);
-}
-
-template <typename T> __device__ __forceinline__ const T *ftab_of(const NvOpDev &op);
-template <> __device__ __forceinline__ const double *ftab_of<double>(const NvOpDev &op) { return op.ftab64; }
-template <> __device__ __forceinline__ const float *ftab_of<float>(const NvOpDev &op) { return op.ftab32; }
-template <typename T> __device__ __forceinline__ const T *cmat_of(const NvOpDev &op);
-template <> __device__ __forceinline__ const double *cmat_of<double>(const NvOpDev &op) { return op.cmat64; }
-template <> __device__ __forceinline__ const float *cmat_of<float>(const NvOpDev &op) { return op.cmat32; }
-
-// ------------------------------------------------------------------------
-// mode digits and the diagonal part
-// ------------------------------------------------------------------------
-// Writes the digits n_k of r into dig[k*kBlock + tid]; returns E(r).
-__device__ __forceinline__ double digits_energy(const NvOpDev &op, int r, uint8_t *dig, int tid) {
-    unsigned rr = (unsigned)r;
-    double e = 0.0;
-    for (int k = op.M - 1; k >= 0; --k) {
-        const unsigned nf = (unsigned)op.nfunc[k];
-        const unsigned q = rr / nf;
-        const unsigned d = rr - q * nf;
-        rr = q;
-        dig[k * kBlock + tid] = (uint8_t)d;
-        e += ((double)d + 0.5) * op.omega[k];
-    }
-    return e;
-}
-
-// The vibrationally diagonal part of H (Source/top.f90:712-756) splits into
-// the state-diagonal E(n) + D_ss(n), precomputed once into op.dg, and the
-// inter-state part D_ss'(n), s != s', evaluated per row when present.
-template <int NS>
-__device__ __forceinline__ void diag_offstate(const NvOpDev &op, const uint8_t *dig, int tid,
-                                              const double (&v)[NS], double (&out)[NS]) {
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-        double a = 0.0;
-#pragma unroll
-        for (int s2 = 0; s2 < NS; ++s2)
-            if (s2 != s) a += op.dconst[s * NS + s2] * v[s2];
-        out[s] += a;
-    }
-    for (int t = 0; t < op.ndterms; ++t) {
-        const NvDiagTerm dt = op.dterms[t];
-        double h = 1.0;
-#pragma unroll
-        for (int j = 0; j < NV_MAXF; ++j)
-            if (j < dt.nf) h *= op.ftab64[dt.code[j] * op.nmax + dig[dt.mode[j] * kBlock + tid]];
-        const double *C = op.dcmat + (size_t)t * NS * NS;
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            double a = 0.0;
-#pragma unroll
-            for (int s2 = 0; s2 < NS; ++s2)
-                if (s2 != s) a += C[s * NS + s2] * v[s2];
-            out[s] += h * a;
-        }
-    }
-}
-
-// out[s] = sum_s' (E + D)(n)_{ss'} v[s'] in FP64.  dig is only read when
-// states are coupled through D.
-template <int NS>
-__device__ __forceinline__ void diag_apply(const NvOpDev &op, int r, const uint8_t *dig, int tid,
-                                           const double (&v)[NS], double (&out)[NS]) {
-#pragma unroll
-    for (int s = 0; s < NS; ++s) out[s] = op.dg[(size_t)s * op.D + r] * v[s];
-    if (op.offstate) diag_offstate<NS>(op, dig, tid, v, out);
-}
 
 // dg[s][r] = E(r) + D_ss(r): harmonic energy, constant term and the Delta=0
 // part of the all-even monomials of the diagonal blocks.
@@ -291,159 +168,6 @@ __device__ __forceinline__ void offdiag_accumulate2(const NvOpDev &op, const TIn
 // basis, whose factor is 0; a negative offset wraps past 2^31) loads 0, so
 // there is no branch per step.
 // ------------------------------------------------------------------------
-typedef float nv_f2 __attribute__((ext_vector_type(2)));
-typedef float nv_f3 __attribute__((ext_vector_type(3)));
-typedef float nv_f4 __attribute__((ext_vector_type(4)));
-
-// Word 3 of the buffer resource: data format 32 (bits 15-18 = 4); the
-// run-time compiled kernels use the same value.
-constexpr int kBufFlags = 0x00020000;
-
-template <int NS, typename TIn> struct XRes;
-
-// One interleaved row as loaded (P = nv_lo_stride values), held apart from its
-// use so that a loop can keep loads of the next iteration in flight.
-template <int P> struct FRow { nv_f4 v[P / 4]; };
-template <> struct FRow<1> { float v; };
-template <> struct FRow<2> { nv_f2 v; };
-template <> struct FRow<3> { nv_f3 v; };
-
-// interleaved FP32 copy, x[r * nv_lo_stride(NS) + s]: one load per row up to
-// four states, 16-byte loads of the states present beyond
-template <int NS> struct XRes<NS, float> {
-    static constexpr unsigned kEl = nv_lo_stride(NS) * 4;
-    __amdgpu_buffer_rsrc_t r;
-    __device__ __forceinline__ XRes(const float *x, int D)
-        : r(__builtin_amdgcn_make_buffer_rsrc((void *)x, (short)0, (int)((unsigned)D * kEl), kBufFlags)) {}
-    template <typename TAcc>
-    __device__ __forceinline__ void fma(unsigned o, TAcc h, TAcc (&w)[NS]) const { fma_so<TAcc>(o, 0u, h, w); }
-    // offset o (per lane) plus so (wave-uniform, a scalar register)
-    template <typename TAcc>
-    __device__ __forceinline__ void fma_so(unsigned o, unsigned so, TAcc h, TAcc (&w)[NS]) const {
-        constexpr int P = nv_lo_stride(NS);
-        if constexpr (P == 1) {
-            const float v = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)o, (int)so, 0));
-            w[0] += h * (TAcc)v;
-        } else if constexpr (P == 2) {
-            const nv_f2 v = __builtin_bit_cast(nv_f2, __builtin_amdgcn_raw_buffer_load_b64(r, (int)o, (int)so, 0));
-#pragma unroll
-            for (int s = 0; s < NS; ++s) w[s] += h * (TAcc)v[s];
-        } else if constexpr (P == 3) {
-            const nv_f3 v = __builtin_bit_cast(nv_f3, __builtin_amdgcn_raw_buffer_load_b96(r, (int)o, (int)so, 0));
-#pragma unroll
-            for (int s = 0; s < NS; ++s) w[s] += h * (TAcc)v[s];
-        } else if constexpr (P == 4) {
-            const nv_f4 v = __builtin_bit_cast(nv_f4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)o, (int)so, 0));
-#pragma unroll
-            for (int s = 0; s < NS; ++s) w[s] += h * (TAcc)v[s];
-        } else {
-#pragma unroll
-            for (int part = 0; part * 4 < NS; ++part) {
-                const nv_f4 v = __builtin_bit_cast(
-                    nv_f4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(o + 16u * part), (int)so, 0));
-#pragma unroll
-                for (int s = part * 4; s < NS && s < part * 4 + 4; ++s) w[s] += h * (TAcc)v[s - part * 4];
-            }
-        }
-    }
-    using Row = FRow<nv_lo_stride(NS)>;
-    __device__ __forceinline__ Row load_so(unsigned o, unsigned so) const {
-        constexpr int P = nv_lo_stride(NS);
-        Row x;
-        if constexpr (P == 1) x.v = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)o, (int)so, 0));
-        else if constexpr (P == 2) x.v = __builtin_bit_cast(nv_f2, __builtin_amdgcn_raw_buffer_load_b64(r, (int)o, (int)so, 0));
-        else if constexpr (P == 3) x.v = __builtin_bit_cast(nv_f3, __builtin_amdgcn_raw_buffer_load_b96(r, (int)o, (int)so, 0));
-        else {
-#pragma unroll
-            for (int part = 0; part < P / 4; ++part)
-                x.v[part] = __builtin_bit_cast(
-                    nv_f4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(o + 16u * part), (int)so, 0));
-        }
-        return x;
-    }
-    template <typename TAcc> static __device__ __forceinline__ void fma_row(const Row &x, TAcc h, TAcc (&w)[NS]) {
-        constexpr int P = nv_lo_stride(NS);
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            if constexpr (P == 1) w[s] += h * (TAcc)x.v;
-            else if constexpr (P <= 3) w[s] += h * (TAcc)x.v[s];
-            else w[s] += h * (TAcc)x.v[s / 4][s % 4];
-        }
-    }
-};
-
-// state-major FP64 vector, x[s * D + r]: one resource per state
-template <int NS> struct XRes<NS, double> {
-    static constexpr unsigned kEl = 8;
-    __amdgpu_buffer_rsrc_t r[NS];
-    __device__ __forceinline__ XRes(const double *x, int D) {
-#pragma unroll
-        for (int s = 0; s < NS; ++s)
-            r[s] = __builtin_amdgcn_make_buffer_rsrc((void *)(x + (size_t)s * D), (short)0, (int)((unsigned)D * 8u),
-                                                     kBufFlags);
-    }
-    template <typename TAcc>
-    __device__ __forceinline__ void fma(unsigned o, TAcc h, TAcc (&w)[NS]) const {
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            const double v = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r[s], (int)o, 0, 0));
-            w[s] += h * (TAcc)v;
-        }
-    }
-};
-
-// interleaved FP64 copy, x[r * nv_lo_stride(NS) + s]: 16-byte loads of two states
-struct F64I {};
-template <int NS> struct XRes<NS, F64I> {
-    static constexpr unsigned kEl = nv_lo_stride(NS) * 8;
-    __amdgpu_buffer_rsrc_t r;
-    __device__ __forceinline__ XRes(const double *x, int D)
-        : r(__builtin_amdgcn_make_buffer_rsrc((void *)x, (short)0, (int)((unsigned)D * kEl), kBufFlags)) {}
-    template <typename TAcc>
-    __device__ __forceinline__ void fma(unsigned o, TAcc h, TAcc (&w)[NS]) const { fma_so<TAcc>(o, 0u, h, w); }
-    template <typename TAcc>
-    __device__ __forceinline__ void fma_so(unsigned o, unsigned so, TAcc h, TAcc (&w)[NS]) const {
-        typedef double nv_d2 __attribute__((ext_vector_type(2)));
-#pragma unroll
-        for (int part = 0; 2 * part < NS; ++part) {
-            if (2 * part + 1 < NS) {
-                const nv_d2 v = __builtin_bit_cast(
-                    nv_d2, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(o + 16u * part), (int)so, 0));
-                w[2 * part] += h * (TAcc)v[0];
-                w[2 * part + 1] += h * (TAcc)v[1];
-            } else {
-                const double v = __builtin_bit_cast(
-                    double, __builtin_amdgcn_raw_buffer_load_b64(r, (int)(o + 16u * part), (int)so, 0));
-                w[2 * part] += h * (TAcc)v;
-            }
-        }
-    }
-    typedef double nv_rd2 __attribute__((ext_vector_type(2)));
-    struct Row {
-        nv_rd2 v[NS / 2];
-        double t;  // the last state when NS is odd
-    };
-    __device__ __forceinline__ Row load_so(unsigned o, unsigned so) const {
-        Row x;
-#pragma unroll
-        for (int part = 0; 2 * part + 1 < NS; ++part)
-            x.v[part] = __builtin_bit_cast(nv_rd2, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(o + 16u * part), (int)so, 0));
-        if constexpr (NS % 2 == 1)
-            x.t = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, (int)(o + 16u * (NS / 2)), (int)so, 0));
-        else
-            x.t = 0.0;
-        return x;
-    }
-    template <typename TAcc> static __device__ __forceinline__ void fma_row(const Row &x, TAcc h, TAcc (&w)[NS]) {
-#pragma unroll
-        for (int s = 0; s + 1 < NS; s += 2) {
-            w[s] += h * (TAcc)x.v[s / 2][0];
-            w[s + 1] += h * (TAcc)x.v[s / 2][1];
-        }
-        if constexpr (NS % 2 == 1) w[NS - 1] += h * (TAcc)x.t;
-    }
-};
-
 // The terms of shape group g; R rows per thread (digits of row q at
 // dig + q * M * kBlock), row q's byte offset in the vector vo[q].  SKIP
 // points the load of a step whose factor is 0 outside the buffer (it then
@@ -568,20 +292,6 @@ __global__ __launch_bounds__(kBlock) void hv_full_kernel(NvOpDev op, const doubl
     diag_apply<NS>(op, r, dig, tid, v, dv);
 #pragma unroll
     for (int s = 0; s < NS; ++s) y[(size_t)s * op.D + r] = dv[s] + (double)acc[s];
-}
-
-__device__ __forceinline__ int64_t slot_of(int64_t i, int64_t nslots) { return i % nslots; }
-
-// A vector element touched once per launch: non-temporal (NT) where the
-// vectors are far larger than the caches, plain otherwise (a vector that fits
-// the Infinity Cache is read again from it by the next kernel).
-template <bool NT, typename T> __device__ __forceinline__ T ld_once(const T *p) {
-    if constexpr (NT) return __builtin_nontemporal_load(p);
-    else return *p;
-}
-template <bool NT, typename T> __device__ __forceinline__ void st_once(T v, T *p) {
-    if constexpr (NT) __builtin_nontemporal_store(v, p);
-    else *p = v;
 }
 
 // Iteration H*v: y = offdiag(H) q_i in TAcc, alpha(i) = q_i . (H q_i) in FP64.
@@ -1134,425 +844,6 @@ __global__ __launch_bounds__(kBlock) void hv2_pass2_kernel(NvOpDev op, LzState s
     }
 }
 
-// ------------------------------------------------------------------------
-// Fast-block H*v (tables in NvFbDev).  A wave owns one block of P <= 64
-// consecutive rows, lane p = row row0 + p: the trailing ("fast") modes vary
-// across the lanes and the slow digits are the same for the whole wave.
-//   1. every distinct slow monomial S: w_S[p] = sum f_S(Delta_s) x[row0 +
-//      Delta_s + p] (wave-uniform factors from a per-wave LDS table, offsets
-//      in the scalar offset field of the buffer loads), mixed into the
-//      channels V_F += C_t w_S of the fast monomials it pairs with (V_1 = y);
-//   2. every channel F > 1: y[p] += sum h_F(p, Delta_f) V_F[p + Delta_f]
-//      through a wave-private LDS row with zero margins;
-//   3. the remaining terms without slow steps, one by one from x[row0 + p].
-// An out-of-basis slow step has factor 0 and reads the first rows of the
-// zero margin that the interleaved copy of x carries, which all such steps
-// share; out-of-block fast neighbours carry factor 0.
-// ------------------------------------------------------------------------
-template <typename T> __device__ __forceinline__ const T *fbtab_of(const NvOpDev &op);
-template <> __device__ __forceinline__ const double *fbtab_of<double>(const NvOpDev &op) { return op.fb.tab64; }
-template <> __device__ __forceinline__ const float *fbtab_of<float>(const NvOpDev &op) { return op.fb.tab32; }
-
-// The four factors h(p, n, -s + 2i) of a slow slot at the wave's digit.
-template <typename T> struct Fb4 { T v[4]; };
-
-// V_c += C_{cm[c]} w for the channels c < NC that the slow monomial d feeds
-// (channel 0 without the middle step when d.excl0).
-template <int NS, typename TAcc, int NC, bool ODD>
-__device__ __forceinline__ void fb_mix(const TAcc *__restrict__ cm, const NvFbS &d, const TAcc (&w)[NS],
-                                       const TAcc (&wf)[NS], TAcc (&V)[NV_FB_NCH][NS]) {
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-        if (d.cm[c] < 0) continue;
-        const TAcc *C = cm + (size_t)d.cm[c] * NS * NS;
-        const bool ex = c == 0 && ODD && d.excl0;
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            TAcc a = V[c][s];
-#pragma unroll
-            for (int s2 = 0; s2 < NS; ++s2) a += C[s * NS + s2] * (ex ? w[s2] : wf[s2]);
-            V[c][s] = a;
-        }
-    }
-}
-
-// The slow monomials [t0, t1) of shape (K0, K1, K2), gathered and mixed into
-// the channels V; vl is the lane's byte offset in its block, rb the byte
-// offset of the block's first row in the padded buffer, fw/fwm the wave's
-// factor rows and their masks of slots inside the basis.  The loop is
-// software-pipelined: monomial t+1's rows are loaded while monomial t's are
-// summed and mixed, each load reusing the registers of the row just summed,
-// so a wave keeps one monomial's loads in flight through the mixing.
-template <int NS, typename TIn, typename TAcc, int NC, int K0, int K1, int K2>
-__device__ __forceinline__ void fb_slow(const NvOpDev &op, const XRes<NS, TIn> &xs, unsigned vl, unsigned rb,
-                                        const TAcc *fw, const int *fwm, int t0, int t1,
-                                        TAcc (&V)[NV_FB_NCH][NS]) {
-    using X = XRes<NS, TIn>;
-    constexpr unsigned kEl = X::kEl;
-    constexpr int J0 = K0 ? K0 : 1, J1 = K1 ? K1 : 1, J2 = K2 ? K2 : 1, J = J0 * J1 * J2;
-    // all stepping slots odd: the middle step is Delta_s = 0
-    constexpr bool odd = K0 > 0 && (K0 & 1) && (K1 == 0 || (K1 & 1)) && (K2 == 0 || (K2 & 1));
-    if (t0 >= t1) return;
-    const TAcc *__restrict__ cm = cmat_of<TAcc>(op);
-    // scalar byte offsets of monomial t's steps, in (i0, i1, i2) order; a step
-    // outside the basis reads the zero margin at offset 0
-    auto offsets = [&](int t, unsigned (&so)[J]) {
-        const NvFbS &d = op.fb.S[t];
-        // slot i of slow slot j is inside the basis when bit i of m_j is set
-        int m0 = 1, m1 = 1, m2 = 1;
-        if constexpr (K0 > 0) m0 = __builtin_amdgcn_readfirstlane(fwm[d.tab[0]]);
-        if constexpr (K1 > 0) m1 = __builtin_amdgcn_readfirstlane(fwm[d.tab[1]]);
-        if constexpr (K2 > 0) m2 = __builtin_amdgcn_readfirstlane(fwm[d.tab[2]]);
-        const unsigned b0 = rb + (unsigned)d.base * kEl;
-        const unsigned ib0 = (unsigned)d.inc[0] * kEl, ib1 = (unsigned)d.inc[1] * kEl,
-                       ib2 = (unsigned)d.inc[2] * kEl;
-#pragma unroll
-        for (int i0 = 0; i0 < J0; ++i0)
-#pragma unroll
-            for (int i1 = 0; i1 < J1; ++i1)
-#pragma unroll
-                for (int i2 = 0; i2 < J2; ++i2) {
-                    unsigned o = rb;
-                    if constexpr (K0 > 0) o = b0 + (unsigned)i0 * ib0;
-                    if constexpr (K1 > 0) o += (unsigned)i1 * ib1;
-                    if constexpr (K2 > 0) o += (unsigned)i2 * ib2;
-                    const bool in = ((m0 >> i0) & (K1 > 0 ? m1 >> i1 : 1) & (K2 > 0 ? m2 >> i2 : 1) & 1) != 0;
-                    so[(i0 * J1 + i1) * J2 + i2] = in ? o : 0u;
-                }
-    };
-    typename X::Row xr[J];
-    {
-        unsigned so[J];
-        offsets(t0, so);
-#pragma unroll
-        for (int k = 0; k < J; ++k) {
-            xr[k] = xs.load_so(vl, so[k]);
-            // loads leave in step order, the order the loop consumes them
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    }
-    for (int t = t0; t < t1; ++t) {
-        const NvFbS &d = op.fb.S[t];
-        Fb4<TAcc> f0, f1, f2;
-        if constexpr (K0 > 0) f0 = *reinterpret_cast<const Fb4<TAcc> *>(fw + d.tab[0] * 4);
-        if constexpr (K1 > 0) f1 = *reinterpret_cast<const Fb4<TAcc> *>(fw + d.tab[1] * 4);
-        if constexpr (K2 > 0) f2 = *reinterpret_cast<const Fb4<TAcc> *>(fw + d.tab[2] * 4);
-        // w: every step but the middle one of an all-odd shape, wc: that one
-        TAcc w[NS], wc[NS];
-#pragma unroll
-        for (int s = 0; s < NS; ++s) w[s] = wc[s] = (TAcc)0;
-        // sums the rows in flight; with next, each row's registers then take
-        // the next monomial's row
-        auto sum_rows = [&](auto next, const unsigned (&sn)[J]) {
-#pragma unroll
-            for (int i0 = 0; i0 < J0; ++i0)
-#pragma unroll
-                for (int i1 = 0; i1 < J1; ++i1)
-#pragma unroll
-                    for (int i2 = 0; i2 < J2; ++i2) {
-                        const int k = (i0 * J1 + i1) * J2 + i2;
-                        TAcc h = (TAcc)1;
-                        if constexpr (K0 > 0) h = f0.v[i0];
-                        if constexpr (K1 > 0) h *= f1.v[i1];
-                        if constexpr (K2 > 0) h *= f2.v[i2];
-                        const bool mid = odd && 2 * i0 + 1 == K0 && (K1 == 0 || 2 * i1 + 1 == K1) &&
-                                         (K2 == 0 || 2 * i2 + 1 == K2);
-                        if (mid) X::template fma_row<TAcc>(xr[k], h, wc);
-                        else X::template fma_row<TAcc>(xr[k], h, w);
-                        if constexpr (decltype(next)::value) {
-                            xr[k] = xs.load_so(vl, sn[k]);
-                            __builtin_amdgcn_sched_barrier(0);
-                        }
-                    }
-        };
-        unsigned sn[J];
-        if (t + 1 < t1) {
-            offsets(t + 1, sn);
-            sum_rows(std::true_type{}, sn);
-        } else {
-            sum_rows(std::false_type{}, sn);
-        }
-        if (d.nd > 0) {
-            TAcc fd = fw[d.dtab[0] * 4];
-            if (d.nd > 1) fd *= fw[d.dtab[1] * 4];
-#pragma unroll
-            for (int s = 0; s < NS; ++s) {
-                w[s] *= fd;
-                if constexpr (odd) wc[s] *= fd;
-            }
-        }
-        // wc stays zero unless the shape has a middle step
-        TAcc wf[NS];
-#pragma unroll
-        for (int s = 0; s < NS; ++s) wf[s] = odd ? w[s] + wc[s] : w[s];
-        fb_mix<NS, TAcc, NC, odd>(cm, d, w, wf, V);
-    }
-}
-
-// y += sum_{steps [s0, s1)} h(p) src[p + stride]: the fast steps of one
-// channel or term over the wave's LDS row vb, src published there first.
-template <int NS, typename TAcc>
-__device__ __forceinline__ void fb_fast(const NvOpDev &op, int s0, int s1, TAcc *vb, int lane, const uint8_t *dig,
-                                        const TAcc *ftab, int tid, const TAcc (&src)[NS], TAcc (&y)[NS]) {
-#pragma unroll
-    for (int s = 0; s < NS; ++s) vb[lane * NS + s] = src[s];
-    __builtin_amdgcn_wave_barrier();
-    const int nmax = op.nmax;
-    for (int k = s0; k < s1; ++k) {
-        const NvStep st = op.fb.steps[k];
-        TAcc h = ftab[st.code[0] * nmax + dig[st.mode[0] * kBlock + tid]];
-#pragma unroll
-        for (int j = 1; j < NV_MAXF; ++j)
-            if (j < st.nf) h *= ftab[st.code[j] * nmax + dig[st.mode[j] * kBlock + tid]];
-        const TAcc *v = vb + (lane + st.stride) * NS;
-#pragma unroll
-        for (int s = 0; s < NS; ++s) y[s] += h * v[s];
-    }
-    __builtin_amdgcn_wave_barrier();
-}
-
-// The off-diagonal part of the wave's block.
-template <int NS, typename TIn, typename TAcc>
-__device__ __forceinline__ void fb_offdiag(const NvOpDev &op, const XRes<NS, TIn> &xs, unsigned vl, unsigned rb,
-                                           int lane, const uint8_t *dig, const TAcc *fw, const int *fwm,
-                                           const TAcc *ftab, int tid, TAcc *vb, TAcc (&y)[NS]) {
-    TAcc V[NV_FB_NCH][NS];
-#pragma unroll
-    for (int c = 0; c < NV_FB_NCH; ++c)
-#pragma unroll
-        for (int s = 0; s < NS; ++s) V[c][s] = (TAcc)0;
-    // phase 0: the slow monomials that feed a channel beyond the first four (degree <= 1);
-    // those channels are complete afterwards and go through LDS, which frees their registers
-    const int *g0 = op.fb.sgrp[0];
-    fb_slow<NS, TIn, TAcc, NV_FB_NCH, 2, 0, 0>(op, xs, vl, rb, fw, fwm, g0[0], g0[1], V);
-    fb_slow<NS, TIn, TAcc, NV_FB_NCH, 0, 0, 0>(op, xs, vl, rb, fw, fwm, g0[7], g0[8], V);
-#pragma unroll
-    for (int c = 4; c < NV_FB_NCH; ++c)
-        if (c < op.fb.nch) fb_fast<NS, TAcc>(op, op.fb.chs[c], op.fb.chs[c + 1], vb, lane, dig, ftab, tid, V[c], y);
-    // phase 1: channels 0..3 (slow degree <= 2)
-    const int *g1 = op.fb.sgrp[1];
-    fb_slow<NS, TIn, TAcc, 4, 2, 0, 0>(op, xs, vl, rb, fw, fwm, g1[0], g1[1], V);
-    fb_slow<NS, TIn, TAcc, 4, 3, 0, 0>(op, xs, vl, rb, fw, fwm, g1[1], g1[2], V);
-    fb_slow<NS, TIn, TAcc, 4, 2, 2, 0>(op, xs, vl, rb, fw, fwm, g1[3], g1[4], V);
-    fb_slow<NS, TIn, TAcc, 4, 0, 0, 0>(op, xs, vl, rb, fw, fwm, g1[7], g1[8], V);
-#pragma unroll
-    for (int c = 1; c < 4; ++c)
-        if (c < op.fb.nch) fb_fast<NS, TAcc>(op, op.fb.chs[c], op.fb.chs[c + 1], vb, lane, dig, ftab, tid, V[c], y);
-    // phase 2: channel 0 only, where most of the slow steps are
-    const int *g2 = op.fb.sgrp[2];
-    fb_slow<NS, TIn, TAcc, 1, 2, 0, 0>(op, xs, vl, rb, fw, fwm, g2[0], g2[1], V);
-    fb_slow<NS, TIn, TAcc, 1, 3, 0, 0>(op, xs, vl, rb, fw, fwm, g2[1], g2[2], V);
-    fb_slow<NS, TIn, TAcc, 1, 4, 0, 0>(op, xs, vl, rb, fw, fwm, g2[2], g2[3], V);
-    fb_slow<NS, TIn, TAcc, 1, 2, 2, 0>(op, xs, vl, rb, fw, fwm, g2[3], g2[4], V);
-    fb_slow<NS, TIn, TAcc, 1, 3, 2, 0>(op, xs, vl, rb, fw, fwm, g2[4], g2[5], V);
-    fb_slow<NS, TIn, TAcc, 1, 2, 3, 0>(op, xs, vl, rb, fw, fwm, g2[5], g2[6], V);
-    fb_slow<NS, TIn, TAcc, 1, 2, 2, 2>(op, xs, vl, rb, fw, fwm, g2[6], g2[7], V);
-    fb_slow<NS, TIn, TAcc, 1, 0, 0, 0>(op, xs, vl, rb, fw, fwm, g2[7], g2[8], V);
-#pragma unroll
-    for (int s = 0; s < NS; ++s) y[s] += V[0][s];
-    if (op.fb.npure > 0) {
-        TAcc xr[NS];
-#pragma unroll
-        for (int s = 0; s < NS; ++s) xr[s] = (TAcc)0;
-        xs.template fma_so<TAcc>(vl, rb, (TAcc)1, xr);
-        const TAcc *__restrict__ cm = cmat_of<TAcc>(op);
-        for (int k = 0; k < op.fb.npure; ++k) {
-            const NvFbPure u = op.fb.pure[k];
-            TAcc fd = (TAcc)1;
-            if (u.nd > 0) fd = fw[u.dtab[0] * 4];
-            if (u.nd > 1) fd *= fw[u.dtab[1] * 4];
-            const TAcc *C = cm + (size_t)u.cm * NS * NS;
-            TAcc v[NS];
-#pragma unroll
-            for (int s = 0; s < NS; ++s) {
-                TAcc a = (TAcc)0;
-#pragma unroll
-                for (int s2 = 0; s2 < NS; ++s2) a += C[s * NS + s2] * xr[s2];
-                v[s] = fd * a;
-            }
-            fb_fast<NS, TAcc>(op, u.s0, u.s1, vb, lane, dig, ftab, tid, v, y);
-        }
-    }
-}
-
-// LDS of the fast-block kernels: factor table, the digits of one row per
-// thread, four wave rows of (64 + 2 halo) lanes x NS values, four wave
-// tables of ntab factor rows x 4 and four of ntab validity masks.
-__host__ __device__ inline size_t fb_lds_layout(const NvOpDev &op, size_t el, size_t *dig_off, size_t *vb_off,
-                                                size_t *fw_off) {
-    const size_t a = ((size_t)op.ncodes * op.nmax * el + 15) & ~(size_t)15;
-    const size_t b = a + (((size_t)op.M * kBlock + 15) & ~(size_t)15);
-    const size_t c = b + ((4 * (size_t)(64 + 2 * op.fb.halo) * op.ns * el + 15) & ~(size_t)15);
-    if (dig_off) *dig_off = a;
-    if (vb_off) *vb_off = b;
-    if (fw_off) *fw_off = c;
-    // factor rows, then one validity mask per row
-    return c + 4 * (size_t)op.fb.ntab * (4 * el + sizeof(int));
-}
-
-// Common prologue: factor table and digits in LDS, the wave's block, its LDS
-// row and its factor rows.
-template <typename TAcc> struct FbWave {
-    const TAcc *ftab;
-    uint8_t *dig;
-    TAcc *vb;
-    const TAcc *fw;
-    const int *fwm;
-    int lane, wave, blk, row0;
-    bool inblk, live;
-};
-template <typename TAcc> __device__ __forceinline__ FbWave<TAcc> fb_prologue(const NvOpDev &op, int b) {
-    extern __shared__ __align__(16) unsigned char lds_raw[];
-    FbWave<TAcc> w;
-    size_t dig_off, vb_off, fw_off;
-    fb_lds_layout(op, sizeof(TAcc), &dig_off, &vb_off, &fw_off);
-    TAcc *ft = reinterpret_cast<TAcc *>(lds_raw);
-    const int nt = op.ncodes * op.nmax;
-    const TAcc *g = ftab_of<TAcc>(op);
-    for (int i = threadIdx.x; i < nt; i += blockDim.x) ft[i] = g[i];
-    w.ftab = ft;
-    w.dig = lds_raw + dig_off;
-    const int tid = threadIdx.x;
-    w.lane = tid & 63;
-    w.wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    w.blk = b * 4 + w.wave;
-    w.inblk = w.blk < op.fb.nblk;
-    {
-        // block t of the sweep: its slow digits in the sweep's mode order
-        int t = w.blk, row0 = 0;
-        for (int j = 0; j < op.fb.nord; ++j) {
-            const int nf = op.fb.ordnf[j];
-            const int q = t / nf;
-            row0 += (t - q * nf) * op.fb.ordshft[j];
-            t = q;
-        }
-        w.row0 = row0;
-    }
-    w.live = w.inblk && w.lane < op.fb.P;
-    if (w.live) digits_energy(op, w.row0 + w.lane, w.dig, tid);
-    else for (int m = 0; m < op.M; ++m) w.dig[m * kBlock + tid] = 0;
-    const int rowlen = (64 + 2 * op.fb.halo) * op.ns;
-    TAcc *vrow = reinterpret_cast<TAcc *>(lds_raw + vb_off) + (size_t)w.wave * rowlen;
-    for (int i = w.lane; i < rowlen; i += 64) vrow[i] = (TAcc)0;
-    w.vb = vrow + (size_t)op.fb.halo * op.ns;
-    __syncthreads();
-    // the wave's factor rows at its slow digits (those of its first lane), and
-    // their masks of slots inside the basis (factor nonzero)
-    TAcc *fw = reinterpret_cast<TAcc *>(lds_raw + fw_off) + (size_t)w.wave * op.fb.ntab * 4;
-    int *fwm = reinterpret_cast<int *>(lds_raw + fw_off + 4 * (size_t)op.fb.ntab * 4 * sizeof(TAcc)) +
-               (size_t)w.wave * op.fb.ntab;
-    const TAcc *tab = fbtab_of<TAcc>(op);
-    for (int k = w.lane; k < op.fb.ntab; k += 64) {
-        const int n = w.dig[op.fb.tabmode[k] * kBlock + w.wave * 64];
-        int m = 0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const TAcc f = tab[((size_t)k * op.nmax + n) * 4 + i];
-            fw[k * 4 + i] = f;
-            m |= (f != (TAcc)0) << i;
-        }
-        fwm[k] = m;
-    }
-    __builtin_amdgcn_wave_barrier();
-    w.fw = fw;
-    w.fwm = fwm;
-    return w;
-}
-
-// Iteration H*v in the fast-block form: y = offdiag(H) q_i, alpha partials.
-// Waves per SIMD the compiler must fit (register budget): 8 for FP32 (60
-// VGPRs) and 4 for FP64 (112).  Four states, 22M rows: FP32 10.7 ms at 6, 7
-// or 8 waves; FP64 23.6 ms at 3 or 4 waves and 28.0 ms at 5, where it spills.
-// (Before the slow monomials were split into phases, the ten channels held 40
-// VGPRs across all of them and the FP32 kernel waited on every load.)
-#ifndef NV_FB_WAVES32
-#define NV_FB_WAVES32 8
-#endif
-#ifndef NV_FB_WAVES64
-#define NV_FB_WAVES64 4
-#endif
-// (Above four states the ten channels of NS values need more registers: the
-// budget follows the state count.)
-constexpr int fb_waves(int ns, int bytes) {
-    return ns <= 4 ? (bytes == 8 ? NV_FB_WAVES64 : NV_FB_WAVES32) : (bytes == 8 ? 1 : 2);
-}
-template <int NS, typename TIn, typename TAcc>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(fb_waves(NS, sizeof(TAcc))))) void
-hv_fb_iter_kernel(NvOpDev op, LzState st) {
-    const int b = xcd_block(blockIdx.x, gridDim.x);
-    const FbWave<TAcc> w = fb_prologue<TAcc>(op, b);
-    const int tid = threadIdx.x;
-    const int64_t it = *st.iter;
-    const double *q = st.V + slot_of(it, st.nslots) * (int64_t)op.N;
-    using TX = typename std::conditional<std::is_same<TIn, F64I>::value, double, TIn>::type;
-    const TX *x = std::is_same<TIn, F64I>::value ? reinterpret_cast<const TX *>(st.v64i)
-                                                 : reinterpret_cast<const TX *>(st.vlo);
-    constexpr int kNsp = nv_lo_stride(NS);
-    constexpr unsigned kEl = XRes<NS, TIn>::kEl;
-    const XRes<NS, TIn> xs(x - (size_t)op.fb.pad * kNsp, op.D + 2 * op.fb.pad);
-    TAcc y[NS];
-#pragma unroll
-    for (int s = 0; s < NS; ++s) y[s] = (TAcc)0;
-    // a lane past the block's P rows loads nothing (offset outside the buffer)
-    const unsigned vl = w.live ? (unsigned)w.lane * kEl : 0x80000000u;
-    const unsigned rb = (unsigned)(w.row0 + op.fb.pad) * kEl;
-    if (w.inblk) fb_offdiag<NS, TIn, TAcc>(op, xs, vl, rb, w.lane, w.dig, w.fw, w.fwm, w.ftab, tid, w.vb, y);
-    double part = 0.0;
-    // q_i, dg and y are touched once per launch (non-temporal on the largest vectors, so that
-    // they do not displace the rows of x that neighbouring blocks gather from L2)
-    auto epilogue = [&](auto nt) {
-        constexpr bool NT = decltype(nt)::value;
-        const int r = w.row0 + w.lane;
-        double v[NS], dv[NS];
-#pragma unroll
-        for (int s = 0; s < NS; ++s) v[s] = ld_once<NT>(&q[(size_t)s * op.D + r]);
-#pragma unroll
-        for (int s = 0; s < NS; ++s) dv[s] = ld_once<NT>(&op.dg[(size_t)s * op.D + r]) * v[s];
-        if (op.offstate) diag_offstate<NS>(op, w.dig, tid, v, dv);
-        TAcc *yo = reinterpret_cast<TAcc *>(st.y);
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            st_once<NT>(y[s], &yo[(size_t)s * op.D + r]);
-            part += v[s] * (dv[s] + (double)y[s]);
-        }
-    };
-    if (w.live) {
-        if (op.stream_nt) epilogue(std::true_type{});
-        else epilogue(std::false_type{});
-    }
-    const double bs = block_sum(part);
-    if (tid == 0) st.partials[b] = bs;
-}
-
-// Standalone y = H x in the fast-block form: xin is the interleaved copy of x
-// (FP32 or FP64, with its margins), x the FP64 vector for the diagonal part.
-template <int NS, typename TIn, typename TAcc>
-__global__ __launch_bounds__(kBlock) void hv_fb_full_kernel(NvOpDev op, const void *__restrict__ xin,
-                                                            const double *__restrict__ x, double *__restrict__ yfull) {
-    const int b = xcd_block(blockIdx.x, gridDim.x);
-    const FbWave<TAcc> w = fb_prologue<TAcc>(op, b);
-    const int tid = threadIdx.x;
-    using TX = typename std::conditional<std::is_same<TIn, F64I>::value, double, TIn>::type;
-    constexpr int kNsp = nv_lo_stride(NS);
-    constexpr unsigned kEl = XRes<NS, TIn>::kEl;
-    const XRes<NS, TIn> xs(reinterpret_cast<const TX *>(xin) - (size_t)op.fb.pad * kNsp, op.D + 2 * op.fb.pad);
-    TAcc y[NS];
-#pragma unroll
-    for (int s = 0; s < NS; ++s) y[s] = (TAcc)0;
-    const unsigned vl = w.live ? (unsigned)w.lane * kEl : 0x80000000u;
-    const unsigned rb = (unsigned)(w.row0 + op.fb.pad) * kEl;
-    if (w.inblk) fb_offdiag<NS, TIn, TAcc>(op, xs, vl, rb, w.lane, w.dig, w.fw, w.fwm, w.ftab, tid, w.vb, y);
-    if (w.live) {
-        const int r = w.row0 + w.lane;
-        double v[NS], dv[NS];
-#pragma unroll
-        for (int s = 0; s < NS; ++s) v[s] = x[(size_t)s * op.D + r];
-        diag_apply<NS>(op, r, w.dig, tid, v, dv);
-#pragma unroll
-        for (int s = 0; s < NS; ++s) yfull[(size_t)s * op.D + r] = dv[s] + (double)y[s];
-    }
-}
-
 // The finishing kernel's sum of parts[0, n) (finish_sum_kernel: strided
 // per-thread sums, then the block tree), in every workgroup of kBlock threads.
 __device__ __forceinline__ double fold_sum(const double *parts, int n) {
@@ -1607,14 +898,6 @@ __global__ __launch_bounds__(kBlock) void lanczos_step_kernel(NvOpDev op, LzStat
     if (st.next_iter && blockIdx.x == 0 && tid == 0) *st.next_iter = it + st.next_inc;
 }
 
-
-// One interleaved row of K values (the H*v input copies), aligned for one
-// wide store where its size allows.
-__host__ __device__ constexpr size_t il_align(size_t b) { return b % 16 == 0 ? 16 : b % 8 == 0 ? 8 : 4; }
-template <typename T, int K> struct alignas(il_align(sizeof(T) * K) < alignof(T) ? alignof(T)
-                                                                                  : il_align(sizeof(T) * K)) IlRow {
-    T v[K];
-};
 
 // update_lanczos (Source/top.f90:646-670): q_i = r / beta(i-1) in place, and
 // the copies of q_i that H*v and re-orthogonalisation read.  A thread takes
@@ -1729,7 +1012,7 @@ constexpr int kShapedMaxStates = NV_MAXS;
 // The shaped kernels serve operators whose terms all have a shape (ordr <= 3),
 // any number of states (up to NV_MAXS), FP64 or FP32, with every row offset inside a 32-bit
 // buffer range; op.tshape = nullptr selects the step-table kernels.
-static bool shaped_ok(const NvOpDev &op, int64_t el) {
+bool shaped_ok(const NvOpDev &op, int64_t el) {
     if (!op.tshape || op.ns > kShapedMaxStates) return false;
     return ((int64_t)op.D + 2 * kBlock) * el < ((int64_t)1 << 31);
 }
@@ -1934,21 +1217,6 @@ static hipError_t step_ns(const NvOpDev &op, int prec, const LzState &st, hipStr
     return hipGetLastError();
 }
 
-#define NV_DISPATCH_NS(fn, ...)                    \
-    switch (op.ns) {                               \
-    case 1: return fn<1>(__VA_ARGS__);             \
-    case 2: return fn<2>(__VA_ARGS__);             \
-    case 3: return fn<3>(__VA_ARGS__);             \
-    case 4: return fn<4>(__VA_ARGS__);             \
-    case 5: return fn<5>(__VA_ARGS__);             \
-    case 6: return fn<6>(__VA_ARGS__);             \
-    case 7: return fn<7>(__VA_ARGS__);             \
-    case 8: return fn<8>(__VA_ARGS__);             \
-    case 9: return fn<9>(__VA_ARGS__);             \
-    case 10: return fn<10>(__VA_ARGS__);           \
-    default: return hipErrorInvalidValue;          \
-    }
-
 template <int NS>
 static hipError_t diag_ns(const NvOpDev &op, double *dg, hipStream_t s) {
     hipLaunchKernelGGL((diag_precompute_kernel<NS>), dim3(hv_blocks(op)), dim3(kBlock), 0, s, op, dg);
@@ -1968,48 +1236,6 @@ hipError_t launch_hv2_full(const NvOpDev &op, int prec, const double *x, const v
     NV_DISPATCH_NS(hv2_ns, op, prec, xin, Z, nullptr, x, y, s)
 }
 
-// ---- fast-block H*v launchers ----
-static size_t hv_fb_lds(const NvOpDev &op, int prec) {
-    return fb_lds_layout(op, prec == 0 ? 8 : 4, nullptr, nullptr, nullptr);
-}
-
-bool hv_fb_use(const NvOpDev &op, int prec) {
-    if (!op.tshape || !op.fb.on || (prec != 0 && prec != 1)) return false;
-    const int64_t el = (int64_t)nv_lo_stride(op.ns) * (prec == 0 ? 8 : 4);
-    return (int64_t)op.D * el >= op.fb_min_bytes && shaped_ok(op, el) && hv_fb_lds(op, prec) <= 64 * 1024 &&
-           ((int64_t)op.D + 2 * (int64_t)op.fb.pad) * el < ((int64_t)1 << 31);
-}
-
-int hv_fb_parts(const NvOpDev &op) { return (op.fb.nblk + 3) / 4; }
-
-template <int NS>
-static hipError_t fb_iter_ns(const NvOpDev &op, int prec, const LzState &st, hipStream_t s) {
-    const size_t lds = hv_fb_lds(op, prec);
-    const unsigned g = (unsigned)hv_fb_parts(op);
-    if (prec == 0)
-        hipLaunchKernelGGL((hv_fb_iter_kernel<NS, F64I, double>), dim3(g), dim3(kBlock), lds, s, op, st);
-    else
-        hipLaunchKernelGGL((hv_fb_iter_kernel<NS, float, float>), dim3(g), dim3(kBlock), lds, s, op, st);
-    return hipGetLastError();
-}
-
-template <int NS>
-static hipError_t fb_full_ns(const NvOpDev &op, int prec, const void *xin, const double *x, double *y,
-                             hipStream_t s) {
-    const size_t lds = hv_fb_lds(op, prec);
-    const unsigned g = (unsigned)hv_fb_parts(op);
-    if (prec == 0)
-        hipLaunchKernelGGL((hv_fb_full_kernel<NS, F64I, double>), dim3(g), dim3(kBlock), lds, s, op, xin, x, y);
-    else
-        hipLaunchKernelGGL((hv_fb_full_kernel<NS, float, float>), dim3(g), dim3(kBlock), lds, s, op, xin, x, y);
-    return hipGetLastError();
-}
-
-hipError_t launch_hv_fb_full(const NvOpDev &op, int prec, const double *x, const void *xin, double *y,
-                             hipStream_t s) {
-    NV_DISPATCH_NS(fb_full_ns, op, prec, xin, x, y, s)
-}
-
 // The iteration H*v runs in the fast-block form when the operator has its
 // tables and the interleaved copy of q_i exists (FP32: LzState::vlo; FP64:
 // LzState::v64i).
@@ -2024,7 +1250,7 @@ static bool hv2_iter(const NvOpDev &op, int prec, const LzState &st) {
 }
 
 static hipError_t hv_iter_any(const NvOpDev &op, int prec, const LzState &st, hipStream_t s) {
-    if (fb_iter(op, prec, st)) NV_DISPATCH_NS(fb_iter_ns, op, prec, st, s)
+    if (fb_iter(op, prec, st)) return launch_hv_fb_iter(op, prec, st, s);
     if (hv2_iter(op, prec, st)) {
         const void *xin = prec == 1 ? st.vlo : (const void *)st.v64i;
         NV_DISPATCH_NS(hv2_ns, op, prec, xin, st.z2, &st, nullptr, nullptr, s)

@@ -29,6 +29,8 @@ struct LzState {
     int64_t ldf = 0;             // N rounded up to even (pairs of FP32 elements load as one)
     double *v64i = nullptr;      // FP64 runs of the shaped generic H*v: q_i interleaved
                                  // [D][nv_lo_stride(ns)], padding zero, written by normalize
+    void *yt = nullptr;          // fast-block H*v with a slab pass: that pass's result, interleaved
+                                 // (hv_slab_bytes)
     void *z2 = nullptr;          // channel scratch of the two-pass H*v (hv2_scratch_bytes), or null
     // Finishing sums folded into their consumers (iterations without re-orthogonalisation on
     // operators with few partials): every workgroup sums fold_in[0, fold_n) in the finishing
@@ -70,8 +72,15 @@ hipError_t launch_cast_f64i(const double *x, double *y, int64_t n, int64_t D, in
 // iteration kernel writes, and y = H x with xin the interleaved copy of x.
 bool hv_fb_use(const NvOpDev &op, int prec);
 int hv_fb_parts(const NvOpDev &op);
-hipError_t launch_hv_fb_full(const NvOpDev &op, int prec, const double *x, const void *xin, double *y,
+hipError_t launch_hv_fb_full(const NvOpDev &op, int prec, const double *x, const void *xin, void *yt, double *y,
                              hipStream_t s);
+hipError_t launch_hv_fb_iter(const NvOpDev &op, int prec, const LzState &st, hipStream_t s);
+// Scratch of its slab pass (LzState::yt, or yt above), 0 when the operator has none.
+size_t hv_slab_bytes(const NvOpDev &op, int prec);
+// Lets its leading pass take more LDS than the default limit (once per context, on its device).
+hipError_t hv_slab_prepare(const NvOpDev &op);
+// Whether rows of el bytes stay within a 32-bit buffer range (and the shaped kernels are selected).
+bool shaped_ok(const NvOpDev &op, int64_t el);
 // The same for the batched H*v (which reads the state-major FP64 vector).
 bool hv_shaped_batch(const NvOpDev &op, int prec);
 // Default of NvOpDev::skip_min_bytes (128 MB).

@@ -5,6 +5,7 @@
 #include <array>
 #include <cmath>
 #include <map>
+#include <set>
 #include <tuple>
 
 namespace nv {
@@ -220,6 +221,16 @@ static void build_two_pass(Operator &op, CodeOf &code_of) {
     op.hv2 = true;
 }
 
+// Whether the slab form takes a term: degree three, slow modes only.
+static bool slab_term(const Term &t, int mf) {
+    int deg = 0;
+    for (int j = 0; j < t.cnt; ++j) {
+        if (t.mode[j] >= mf) return false;
+        deg += t.pow[j];
+    }
+    return deg == 3;
+}
+
 // Tables of the fast-block H*v (NvFbDev).  The fast modes are the trailing
 // modes whose basis product P is at most 64 (one block of P rows per wave);
 // the form needs 33 <= P <= 64, a slow mode, ordr <= 3, at most NV_FB_NCH
@@ -353,6 +364,7 @@ static void build_fast_block(Operator &op, CodeOf &code_of, std::vector<std::arr
     }
     for (size_t c = chkeys.size(); c < NV_FB_NCH; ++c) op.fb_chs[c + 1] = op.fb_chs[c];
     // slow monomials
+    std::set<Key> slab_keys;
     std::vector<std::vector<NvFbS>> byshape(NV_FB_NSLOW);
     std::map<Key, std::pair<int, int>> sindex;  // slow key -> (shape, position)
     int64_t pad = 0;
@@ -403,6 +415,7 @@ static void build_fast_block(Operator &op, CodeOf &code_of, std::vector<std::arr
         }
         NvFbS &S = byshape[it->second.first][it->second.second];
         S.cm[ch->second] = op.term_dev[ti];
+        if (x.fkey.empty() && slab_term(t, mf)) slab_keys.insert(x.skey);
         S.nchk = std::max<int32_t>(S.nchk, ch->second + 1);
         if (ch->second == 0 && t.diag) S.excl0 = 1;
     }
@@ -412,18 +425,30 @@ static void build_fast_block(Operator &op, CodeOf &code_of, std::vector<std::arr
     static const bool kPhaseShape[3][NV_FB_NSLOW] = {{1, 0, 0, 0, 0, 0, 0, 1},
                                                      {1, 1, 0, 1, 0, 0, 0, 1},
                                                      {1, 1, 1, 1, 1, 1, 1, 1}};
+    // (a monomial of degree three over the slow modes feeds y alone: phase 2, after the others
+    // of its shape, where the slab form cuts it off)
+    std::vector<std::vector<char>> inslab(NV_FB_NSLOW);
+    for (int q = 0; q < NV_FB_NSLOW; ++q) inslab[q].assign(byshape[q].size(), 0);
+    for (auto &kv : sindex) inslab[kv.second.first][kv.second.second] = (char)slab_keys.count(kv.first);
     for (int ph = 0; ph < 3; ++ph) {
         for (int q = 0; q < NV_FB_NSLOW; ++q) {
             op.fb_sgrp[ph][q] = (int32_t)op.fb_S.size();
-            for (auto &S : byshape[q]) {
-                const int sp_ = S.nchk > 4 ? 0 : (S.nchk > 1 ? 1 : 2);
-                if (sp_ != ph) continue;
-                if (!kPhaseShape[ph][q]) return;
-                op.fb_S.push_back(S);
+            for (int last = 0; last < 2; ++last) {
+                for (size_t k = 0; k < byshape[q].size(); ++k) {
+                    const NvFbS &S = byshape[q][k];
+                    const int sp_ = S.nchk > 4 ? 0 : (S.nchk > 1 ? 1 : 2);
+                    if (sp_ != ph || inslab[q][k] != last) continue;
+                    if (!kPhaseShape[ph][q]) return;
+                    op.fb_S.push_back(S);
+                }
+                if (ph == 2 && last == 0) op.slab_s2end[q] = (int32_t)op.fb_S.size();
             }
         }
         op.fb_sgrp[ph][NV_FB_NSLOW] = (int32_t)op.fb_S.size();
     }
+    for (auto &S : op.fb_S)
+        for (int c = 0; c < NV_FB_NCH; ++c)
+            if (S.cm[c] >= 0) S.cmask |= 1 << c;
     op.fb_nch = (int32_t)chkeys.size();
     op.fb_mf = mf;
     op.fb_P = (int32_t)P;
@@ -431,6 +456,220 @@ static void build_fast_block(Operator &op, CodeOf &code_of, std::vector<std::arr
     // out-of-basis slow steps read the first 64 rows of the margin
     op.fb_pad = (int32_t)std::max<int64_t>(pad, 64);
     op.fb = true;
+}
+
+// Tables of the slab H*v (NvSlabDev): after build_fast_block.  At most four
+// states; L is as many trailing slow modes (up to NV_SLAB_NL) as keep points
+// times rows within a workgroup.
+static void build_slab(Operator &op) {
+    op.slab = false;
+    op.slab_G.clear();
+    op.slab_S.clear();
+    op.slab_tabdiv.clear();
+    op.slab_tab.clear();
+    op.slab_ltab.clear();
+    for (int k = 0; k < NV_SLAB_NL; ++k) op.slab_c3[k] = -1;
+    for (int k = 0; k < 6; ++k) op.slab_c21[k] = -1;
+    op.slab_c111 = -1;
+    op.slab_kl = 0;
+    op.slab_ktab.clear();
+    for (auto &v : op.slab_k3) v = -1;
+    for (auto &v : op.slab_k21) v = -1;
+    for (auto &v : op.slab_k111) v = -1;
+    if (!op.fb || op.ns > 4) return;
+    const int mf = op.fb_mf;
+    std::vector<size_t> mine;
+    for (size_t ti = 0; ti < op.terms.size(); ++ti)
+        if (op.term_dev[ti] >= 0 && slab_term(op.terms[ti], mf)) mine.push_back(ti);
+    if (mine.empty()) return;
+    // (the sweep that goes with the slab pass has no monomial of degree three left over the slow modes)
+    for (int q : {2, 4, 5, 6})
+        if (op.slab_s2end[q] != op.fb_sgrp[2][q]) return;
+    // rows per workgroup: a thread's rows are the smallest divisor of P with at least 64 bytes of
+    // rows, and it takes two such runs (a 128-byte line) when they divide P
+    const int P = op.fb_P, nsp = nv_lo_stride((int)op.ns);
+    auto rows = [&](int el, int32_t &r, int32_t &R) {
+        r = P;
+        for (int q = 1; q < P; ++q)
+            if (P % q == 0 && q * nsp * el >= 64) {
+                r = q;
+                break;
+            }
+        R = 1;
+        if (r * nsp * el < 128 && P % (2 * r) == 0) {
+            R = 2;
+            r *= 2;
+        }
+    };
+    rows(8, op.slab_r64, op.slab_R64);
+    rows(4, op.slab_r32, op.slab_R32);
+    // LDS of a workgroup (hv_slab_kernel): two buffers of a row per thread and run, the factor tables
+    auto fits = [&](int64_t points, int nl, int r, int R, int el) {
+        const int64_t t = (points * (r / R) + 63) / 64 * 64;
+        const int64_t tabs = (int64_t)3 * (mf - nl) * (4 * el + 4) + (int64_t)nl * op.nmax * 9 * el + 32;
+        // (two rows per thread: 640 threads of FP32 and 320 of FP64 leave the registers they need)
+        return t <= (R == 1 ? 1024 : el == 4 ? 640 : 320) && 2 * R * t * op.ns * el + tabs <= 64 * 1024;
+    };
+    int gl = mf;
+    int64_t pts = 1;
+    while (gl > 0 && mf - gl < NV_SLAB_NL) {
+        const int64_t np = pts * op.nfunc[gl - 1];
+        if (!fits(np, mf - gl + 1, op.slab_r64, op.slab_R64, 8) ||
+            !fits(np, mf - gl + 1, op.slab_r32, op.slab_R32, 4))
+            break;
+        pts = np;
+        --gl;
+    }
+    if (gl == mf) return;
+    op.slab_gl = gl;
+    op.slab_nl = mf - gl;
+    op.slab_pts = (int32_t)pts;
+    int64_t gpts = 1;
+    for (int k = 0; k < gl; ++k) gpts *= op.nfunc[k];
+    op.slab_gpts = (int32_t)gpts;
+    auto elem = [&](int m, int p, int64_t n, int d) {
+        const int64_t n2 = n + d;
+        if (n >= op.nfunc[m] || n2 < 0 || n2 >= op.nfunc[m]) return 0.0;
+        return hoelem(p, std::min(n, n2), std::abs(d), op.quirks);
+    };
+    auto push_rows = [&](int m, std::vector<double> &to) {
+        for (int64_t n = 0; n < op.nmax; ++n)
+            for (int p = 1; p <= 3; ++p)
+                for (int i = 0; i <= p; ++i) to.push_back(elem(m, p, n, -p + 2 * i));
+    };
+    for (int l = 0; l < op.slab_nl; ++l) push_rows(gl + l, op.slab_ltab);
+    // the leading pass: two to NV_LEAD_NL modes of G whose points, at 64 bytes of rows or more, fit
+    // one CU's LDS with their factors
+    op.slab_kr64 = op.slab_r64 / op.slab_R64;
+    op.slab_kr32 = op.slab_r32 / op.slab_R32;
+    {
+        int64_t kp = 1;
+        int kl = 0;
+        while (kl < gl && kl < NV_LEAD_NL) {
+            const int64_t np = kp * op.nfunc[kl];
+            const int64_t b64 = np * op.slab_kr64 * op.ns * 8 + (int64_t)(kl + 1) * op.nmax * 72 + 16;
+            const int64_t b32 = np * op.slab_kr32 * op.ns * 4 + (int64_t)(kl + 1) * op.nmax * 36 + 16;
+            if (std::max(b64, b32) > NV_LEAD_LDS) break;
+            kp = np;
+            ++kl;
+        }
+        if (kl >= 2) {
+            op.slab_kl = kl;
+            op.slab_kpts = (int32_t)kp;
+            for (int k = 0; k < kl; ++k) push_rows(k, op.slab_ktab);
+        }
+    }
+    std::map<std::pair<int, int>, int> tabs;
+    auto tab_of = [&](int m, int p) {
+        auto key = std::make_pair(m, p);
+        auto it = tabs.find(key);
+        if (it != tabs.end()) return it->second;
+        const int k = (int)tabs.size();
+        tabs[key] = k;
+        int64_t div = 1;
+        for (int j = m + 1; j < gl; ++j) div *= op.nfunc[j];
+        op.slab_tabdiv.push_back((int32_t)div);
+        op.slab_tabdiv.push_back((int32_t)op.nfunc[m]);
+        for (int64_t n = 0; n < op.nmax; ++n)
+            for (int i = 0; i < 4; ++i) op.slab_tab.push_back(i <= p ? elem(m, p, n, -p + 2 * i) : 0.0);
+        return k;
+    };
+    static const int kSlow[NV_FB_NSLOW - 1][3] = {{2, 0, 0}, {3, 0, 0}, {4, 0, 0}, {2, 2, 0},
+                                                  {3, 2, 0}, {2, 3, 0}, {2, 2, 2}};
+    typedef std::vector<std::pair<int, int>> Key;
+    struct Tmp { int shape; NvSlabG g; };
+    std::vector<Tmp> gs;
+    std::map<Key, int> gindex;
+    std::vector<std::vector<NvFbS>> deg3(NV_FB_NSLOW);
+    for (size_t ti : mine) {
+        const Term &t = op.terms[ti];
+        const int cm = op.term_dev[ti];
+        Key gk, lk;  // (mode, pow); L modes numbered from gl
+        for (int j = 0; j < t.cnt; ++j) {
+            if (t.mode[j] < gl) gk.push_back({t.mode[j], t.pow[j]});
+            else lk.push_back({t.mode[j] - gl, t.pow[j]});
+        }
+        std::sort(gk.begin(), gk.end());
+        std::sort(lk.begin(), lk.end());
+        if (gk.empty()) {
+            if (lk.size() == 1) op.slab_c3[lk[0].first] = cm;
+            else if (lk.size() == 3) op.slab_c111 = cm;
+            else {
+                const int k = lk[0].second == 2 ? lk[0].first : lk[1].first;
+                const int l = lk[0].second == 2 ? lk[1].first : lk[0].first;
+                op.slab_c21[k * 2 + (l < k ? l : l - 1)] = cm;
+            }
+            continue;
+        }
+        if (lk.empty() && gk.back().first < op.slab_kl) {
+            if (gk.size() == 1) op.slab_k3[gk[0].first] = cm;
+            else if (gk.size() == 3) op.slab_k111[gk[0].first + gk[1].first + gk[2].first - 3] = cm;
+            else {
+                const int k = gk[0].second == 2 ? gk[0].first : gk[1].first;
+                const int l = gk[0].second == 2 ? gk[1].first : gk[0].first;
+                op.slab_k21[k * (NV_LEAD_NL - 1) + (l < k ? l : l - 1)] = cm;
+            }
+            continue;
+        }
+        // steps of the G part
+        int64_t base = 0;
+        int32_t inc[3] = {0, 0, 0}, tab[3] = {0, 0, 0};
+        int k3[3] = {0, 0, 0};
+        for (size_t j = 0; j < gk.size(); ++j) {
+            const int m = gk[j].first, p = gk[j].second;
+            base -= (int64_t)p * op.shft[m];
+            inc[j] = (int32_t)(2 * op.shft[m]);
+            tab[j] = tab_of(m, p);
+            k3[j] = p + 1;
+        }
+        int q = 0;
+        while (k3[0] != kSlow[q][0] || k3[1] != kSlow[q][1] || k3[2] != kSlow[q][2]) ++q;
+        if (lk.empty()) {
+            NvFbS S{};
+            S.base = (int32_t)base;
+            for (int j = 0; j < 3; ++j) { S.inc[j] = inc[j]; S.tab[j] = tab[j]; }
+            for (int c = 0; c < NV_FB_NCH; ++c) S.cm[c] = -1;
+            S.cm[0] = cm;
+            S.nchk = 1;
+            deg3[q].push_back(S);
+            continue;
+        }
+        auto it = gindex.find(gk);
+        if (it == gindex.end()) {
+            Tmp x;
+            x.shape = q;
+            x.g.base = (int32_t)base;
+            for (int j = 0; j < 3; ++j) {
+                x.g.inc[j] = inc[j];
+                x.g.tab[j] = tab[j];
+                x.g.c1[j] = x.g.c2[j] = x.g.c11[j] = -1;
+            }
+            gindex[gk] = (int)gs.size();
+            gs.push_back(x);
+            it = gindex.find(gk);
+        }
+        NvSlabG &g = gs[it->second].g;
+        if (lk.size() == 2) g.c11[lk[0].first + lk[1].first - 1] = cm;  // (0,1) (0,2) (1,2)
+        else if (lk[0].second == 2) g.c2[lk[0].first] = cm;
+        else g.c1[lk[0].first] = cm;
+    }
+    static const int kGShape[3] = {0, 1, 3};  // (2), (3), (2,2)
+    for (int z = 0; z < 3; ++z) {
+        op.slab_ggrp[z] = (int32_t)op.slab_G.size();
+        for (auto &x : gs)
+            if (x.shape == kGShape[z]) op.slab_G.push_back(x.g);
+    }
+    op.slab_ggrp[3] = (int32_t)op.slab_G.size();
+    for (int q = 0; q < NV_FB_NSLOW; ++q) {
+        op.slab_sgrp[q] = (int32_t)op.slab_S.size();
+        for (auto &S : deg3[q]) op.slab_S.push_back(S);
+    }
+    op.slab_sgrp[NV_FB_NSLOW] = (int32_t)op.slab_S.size();
+    // out-of-basis steps read from the start of the margin, every row of the workgroup
+    op.fb_pad = (int32_t)std::max<int64_t>(op.fb_pad, pts * P);
+    op.slab_steps = 0;
+    for (size_t ti : mine) op.slab_steps += op.dev_terms[op.term_dev[ti]].nsteps;
+    op.slab = true;
 }
 
 bool build_operator(const nv_problem &pr, Operator &op, std::string &err) {
@@ -694,6 +933,7 @@ bool build_operator(const nv_problem &pr, Operator &op, std::string &err) {
             for (int i = 0; i < 4; ++i)
                 if (fb_tabcodes[k][i] >= 0)
                     op.fb_tab[(k * op.nmax + n) * 4 + i] = op.ftab[(size_t)fb_tabcodes[k][i] * op.nmax + n];
+    build_slab(op);
 
     // ---- start-vector data ----
     op.neworigin = pr.neworigin;

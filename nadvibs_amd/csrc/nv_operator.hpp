@@ -71,6 +71,22 @@ struct Operator {
     std::vector<NvStep> fb_steps;          // fast steps of the channels, then of the pure terms
     std::vector<NvFbPure> fb_pure;
 
+    // slab H*v tables (see NvSlabDev); fb_S lists the terms it takes last in each phase-2 group
+    bool slab = false;
+    int64_t slab_steps = 0;              // steps of the terms it takes
+    int32_t slab_gl = 0, slab_nl = 0, slab_gpts = 0, slab_pts = 0, slab_r64 = 0, slab_r32 = 0, slab_R64 = 1,
+            slab_R32 = 1;
+    int32_t slab_ggrp[4] = {0}, slab_sgrp[NV_FB_NSLOW + 1] = {0}, slab_s2end[NV_FB_NSLOW] = {0};
+    int32_t slab_c3[NV_SLAB_NL] = {0}, slab_c21[6] = {0}, slab_c111 = -1;
+    std::vector<NvSlabG> slab_G;
+    std::vector<NvFbS> slab_S;
+    std::vector<int32_t> slab_tabdiv;    // [ntab][2]
+    std::vector<double> slab_tab;        // [ntab][nmax][4]
+    std::vector<double> slab_ltab;       // [nl][nmax][9]
+    int32_t slab_kl = 0, slab_kpts = 0, slab_kr64 = 1, slab_kr32 = 1;
+    int32_t slab_k3[NV_LEAD_NL] = {0}, slab_k21[NV_LEAD_NL * (NV_LEAD_NL - 1)] = {0}, slab_k111[4] = {0};
+    std::vector<double> slab_ktab;       // [kl][nmax][9]
+
     // start vector data
     int32_t neworigin = 0;
     std::vector<double> statew, bomega, dvec, tmat;
