@@ -989,7 +989,7 @@ int32_t nv_partial_orthog(nv_ctx *c, int64_t it) {
     int32_t rc = check_iter(c, it);
     if (rc) return rc;
     if (c->opts.reorthog <= 0 || it <= 1) return NV_OK;
-    NV_HIP(c, nv::pro_partial_orthog(c->pro, c->dev, c->st, c->stream));
+    NV_HIP(c, nv::pro_partial_orthog(c->pro, c->dev, c->st, true, c->stream));
     return NV_OK;
 }
 
@@ -1006,14 +1006,15 @@ static hipError_t enqueue_iteration(nv_ctx *c, int pro, int check, bool set = tr
     if (pro && !check && nv::pro_fusable(c->pro)) {
         // beta, the omega recurrence and the range decision in one workgroup
         if (e == hipSuccess) e = nv::launch_lanczos_step_only(c->dev, c->opts.prec, c->st, c->stream);
-        if (e == hipSuccess) e = nv::pro_step_fused(c->pro, c->dev, c->st, nv::hv_blocks(c->dev), c->stream);
+        if (e == hipSuccess) e = nv::pro_step_fused(c->pro, c->dev, c->st, c->st.partials, nv::hv_blocks(c->dev),
+                                                      true, c->stream);
         return e;
     }
     if (e == hipSuccess)
         e = nv::launch_lanczos_step(c->dev, c->opts.prec, c->st, c->stream, advance ? c->d_iter : nullptr);
     if (pro) {
         if (e == hipSuccess) e = nv::pro_set_omega(c->pro, c->dev, c->st, check, c->stream);
-        if (e == hipSuccess) e = nv::pro_partial_orthog(c->pro, c->dev, c->st, c->stream);
+        if (e == hipSuccess) e = nv::pro_partial_orthog(c->pro, c->dev, c->st, true, c->stream);
     }
     return e;
 }
@@ -1077,6 +1078,42 @@ static hipError_t enqueue_folded_batch(nv_ctx *c) {
     return e;
 }
 
+// One iteration with re-orthogonalisation under the same limits, without its
+// counter and finishing launches (set_iter, alpha, beta: 13 us of a 1.38M-element
+// iteration's 45 us of kernels that do next to nothing, against 3 us more in
+// the step, whose workgroups each sum 1,350 partials): normalize takes
+// iteration *d_iter + 1 and publishes it in d_iter + 1 for the kernels after
+// it, and the step advances d_iter; the step sums alpha, and normalize the
+// Gram-Schmidt update's |r| when the iteration before listed vectors.  After
+// the last one of a run pro_finish_beta leaves the state of the per-call path.
+static hipError_t enqueue_folded_pro(nv_ctx *c, int check) {
+    hipStream_t s = c->stream;
+    double *bparts = c->st.partials + kFoldMax;
+    nv::LzState st = c->st;
+    st.iter = c->d_iter + 1;
+    nv::LzState sn = c->st;
+    sn.iter_add = 1;
+    sn.iter_pub = c->d_iter + 1;
+    sn.fold_in = c->st.partials;
+    sn.fold_n = nv::pro_axpy_parts(c->op.N);
+    sn.fold_cond = c->pro.d.njl;
+    hipError_t e = nv::launch_normalize(c->dev, c->opts.prec, sn, s);
+    if (e == hipSuccess) e = launch_hv_iter_nofinish(c, st);
+    nv::LzState ss = st;
+    ss.fold_in = st.partials;
+    ss.fold_n = hv_iter_nparts(c);
+    ss.fold_out = bparts;
+    ss.next_iter = c->d_iter;
+    if (e == hipSuccess) e = nv::launch_lanczos_step_only(c->dev, c->opts.prec, ss, s);
+    if (e != hipSuccess) return e;
+    const int nstep = nv::hv_blocks(c->dev);
+    if (!check && nv::pro_fusable(c->pro)) return nv::pro_step_fused(c->pro, c->dev, st, bparts, nstep, false, s);
+    e = nv::launch_finish_sum(bparts, nstep, c->st.beta, st.iter, 1, s);
+    if (e == hipSuccess) e = nv::pro_set_omega(c->pro, c->dev, st, check, s);
+    if (e == hipSuccess) e = nv::pro_partial_orthog(c->pro, c->dev, st, false, s);
+    return e;
+}
+
 static hipError_t iteration_graph(nv_ctx *c, int kind, hipGraphExec_t *out) {
     if (c->graphs[kind]) {
         *out = c->graphs[kind];
@@ -1091,6 +1128,8 @@ static hipError_t iteration_graph(nv_ctx *c, int kind, hipGraphExec_t *out) {
     else if (kind == 3)
         for (int64_t k = 0; k < kIterBatch && e2 == hipSuccess; ++k)
             e2 = enqueue_iteration(c, 0, 0, k == 0, k + 1 < kIterBatch);
+    else if (kind >= 1 && fold_ok(c))
+        e2 = enqueue_folded_pro(c, kind == 2);
     else
         e2 = enqueue_iteration(c, kind >= 1, kind == 2);
     e = hipStreamEndCapture(c->stream, &g);
@@ -1108,6 +1147,7 @@ int32_t nv_lanczos_run(nv_ctx *c, int64_t iiter, int64_t niter) {
     if (niter > c->opts.niter) return fail(c, NV_ERR_ARG, "niter beyond the initialised run");
     NV_HIP(c, hipSetDevice(c->device));
     const bool orthog = c->opts.reorthog > 0;
+    bool open_beta = false;  // the last iteration left its beta to the next
     for (int64_t i = iiter; i <= niter; ++i) {
         // the first iteration of a call and profiled runs go through the
         // per-call path, which sets the device iteration counter that the
@@ -1140,8 +1180,10 @@ int32_t nv_lanczos_run(nv_ctx *c, int64_t iiter, int64_t niter) {
         NV_HIP(c, hipGraphLaunch(ge, c->stream));
         c->next_update = i + 1;
         c->last_iter = i;
+        open_beta = kind >= 1 && fold_ok(c);
         NV_HIP(c, save_checkpoint(c, i));
     }
+    if (open_beta) NV_HIP(c, nv::pro_finish_beta(c->pro, c->op.N, c->st, c->stream));
     return NV_OK;
 }
 

@@ -905,10 +905,11 @@ __global__ __launch_bounds__(kBlock) void lanczos_step_kernel(NvOpDev op, LzStat
 template <int NS, typename TIn, bool NT>
 __global__ __launch_bounds__(kBlock) void normalize_rows_kernel(int64_t N, int64_t D, LzState st) {
     constexpr int NSP = nv_lo_stride(NS);
-    const int64_t it = *st.iter;
+    const int64_t it = *st.iter + st.iter_add;
+    if (st.iter_pub && blockIdx.x == 0 && threadIdx.x == 0) *st.iter_pub = it;
     double *q = st.V + slot_of(it, st.nslots) * N;
     double bprev;
-    if (st.fold_in) {
+    if (st.fold_in && (!st.fold_cond || *st.fold_cond != 0)) {
         bprev = sqrt(fold_sum(st.fold_in, st.fold_n));
         if (blockIdx.x == 0 && threadIdx.x == 0) st.beta[it - 1] = bprev;
     } else {

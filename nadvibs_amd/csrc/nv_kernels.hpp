@@ -41,6 +41,11 @@ struct LzState {
     double *fold_out = nullptr;       // step: its beta partials go here instead of partials
     int64_t *next_iter = nullptr;     // step: block 0 stores it + next_inc there (a counter that no
     int32_t next_inc = 0;             //   workgroup of the same launch reads)
+    // Iterations with re-orthogonalisation: normalize takes iteration *iter + iter_add, block 0 stores
+    // it at iter_pub, and fold_in counts only when *fold_cond is not zero (else beta[it-1] stands).
+    int32_t iter_add = 0;
+    int64_t *iter_pub = nullptr;
+    const int32_t *fold_cond = nullptr;
 };
 
 // counters[] slots

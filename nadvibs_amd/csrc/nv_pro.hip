@@ -41,6 +41,28 @@ __device__ void recur_body(const ProDev &p, const LzState &st, double bi) {
     const int64_t it = *st.iter;
     double *o1 = p.omega, *o2 = p.omega + p.ostride;
     const uint64_t base = (uint64_t)p.meta[2];
+    if (it <= (int64_t)blockDim.x) {
+        // an index per thread: the new row stays in a register until every thread has read the old ones
+        const int64_t k = 1 + threadIdx.x;
+        double was = 0.0, now = 0.0;
+        if (k <= it) was = o2[k];
+        if (k < it)
+            now = (1 / bi) * (st.beta[k] * o2[k + 1] + (st.alpha[k] - st.alpha[it]) * was +
+                              st.beta[k - 1] * o2[k - 1] - st.beta[it - 1] * o1[k]) +
+                  p.eps * (st.beta[k] + bi) * (p.noise * noise_gauss(p.seed, base + (uint64_t)k, 0.3));
+        else if (k == it)
+            now = p.noise * noise_gauss(p.seed, base, 0.6) * p.epsn * st.beta[1] / bi;
+        __syncthreads();
+        if (k <= it) {
+            o2[k] = now;
+            o1[k] = was;
+        }
+        if (threadIdx.x == 0) {
+            if (it < p.niter) o2[it + 1] = 1.0;
+            p.meta[2] = (int64_t)base + it;
+        }
+        return;
+    }
     if (threadIdx.x == 0) {
         if (it < p.niter) o2[it + 1] = 1.0;
         o1[it] = p.noise * noise_gauss(p.seed, base, 0.6) * p.epsn * st.beta[1] / bi;
@@ -326,6 +348,14 @@ __device__ void decide_body(const ProDev &p, const LzState &st) {
             if (w < p.eta) smallm |= 1u << (i - i0);
             if (w >= p.seps) bigm |= 1u << (i - i0);
         }
+        if (!__syncthreads_or((int)bigm)) {
+            // no large index, so no range: most iterations end here
+            if (threadIdx.x == 0) {
+                p.meta[1] = 0;
+                *p.njl = 0;
+            }
+            return;
+        }
         const int64_t sbase = scan_excl(__popc(smallm), &tot);
         const int64_t m = tot;  // number of small indices; gaps 0..m
         for (int64_t g = threadIdx.x; g <= m; g += kDecide) act[g] = 0;
@@ -484,6 +514,8 @@ __global__ __launch_bounds__(kBlock) void pro_axpy_kernel(int64_t N, ProDev p, L
     if (threadIdx.x == 0) st.partials[blockIdx.x] = b;
 }
 
+int pro_axpy_parts(int64_t N) { return (int)std::min<int64_t>((N + kBlock - 1) / kBlock, 4096); }
+
 // beta(it) = |residual| after the update (only when vectors were listed).
 __global__ __launch_bounds__(kBlock) void pro_beta_kernel(ProDev p, LzState st, int nparts) {
     if (*p.njl == 0) return;
@@ -498,14 +530,19 @@ __global__ __launch_bounds__(kBlock) void pro_beta_kernel(ProDev p, LzState st, 
 // lanczos_step's block partials (summed as finish_sum_kernel sums them: a
 // 256-thread strided pass, then four wave sums in order), the omega
 // recurrence and the range decision -- three launches of the per-call path.
-__global__ __launch_bounds__(kDecide) void pro_step_kernel(ProDev p, LzState st, int nparts) {
+// A chain of dependent loads and barriers: 11.1 us at 500 iterations with the
+// omega rows swapped through memory and the range scans always run, 7.6 us
+// with an index per thread held in a register and the scans left out when no
+// index is large.
+__global__ __launch_bounds__(kDecide) void pro_step_kernel(ProDev p, LzState st, const double *bparts,
+                                                       int nparts) {
     __shared__ double red[kBlock / 64];
     __shared__ double sh_beta;
     const int64_t it = *st.iter;
     double v = 0.0;
     if (threadIdx.x < kBlock) {
 #pragma unroll 8
-        for (int i = threadIdx.x; i < nparts; i += kBlock) v += st.partials[i];
+        for (int i = threadIdx.x; i < nparts; i += kBlock) v += bparts[i];
     }
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
     if (threadIdx.x < kBlock && (threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
@@ -655,35 +692,42 @@ hipError_t pro_set_omega(ProState &ps, const NvOpDev &dev, const LzState &st, in
     return e;
 }
 
-// The dots and the update of the decided list, and beta after it.
-static hipError_t orthog_apply(const ProState &ps, const NvOpDev &dev, const LzState &st, hipStream_t s) {
+hipError_t pro_finish_beta(const ProState &ps, int64_t N, const LzState &st, hipStream_t s) {
+    hipLaunchKernelGGL(pro_beta_kernel, dim3(1), dim3(kBlock), 0, s, ps.d, st, pro_axpy_parts(N));
+    return hipGetLastError();
+}
+
+// The dots and the update of the decided list, and with `beta` beta after it.
+static hipError_t orthog_apply(const ProState &ps, const NvOpDev &dev, const LzState &st, bool beta,
+                               hipStream_t s) {
     const ProDev &p = ps.d;
     hipError_t e = multidot(ps, dev.N, st, p.jlist, p.njl, 0, 0, 1, s);  // count = list length
     if (e != hipSuccess) return e;
     const int64_t N = dev.N;
-    int g = (int)std::min<int64_t>((N + kBlock - 1) / kBlock, 4096);
+    const int g = pro_axpy_parts(N);
     if (st.Vf)
         hipLaunchKernelGGL(pro_axpy_kernel<float>, dim3(g), dim3(kBlock), 0, s, N, p, st);
     else
         hipLaunchKernelGGL(pro_axpy_kernel<double>, dim3(g), dim3(kBlock), 0, s, N, p, st);
-    hipLaunchKernelGGL(pro_beta_kernel, dim3(1), dim3(kBlock), 0, s, p, st, g);
-    return hipGetLastError();
+    e = hipGetLastError();
+    return e != hipSuccess || !beta ? e : pro_finish_beta(ps, N, st, s);
 }
 
-hipError_t pro_partial_orthog(ProState &ps, const NvOpDev &dev, const LzState &st, hipStream_t s) {
+hipError_t pro_partial_orthog(ProState &ps, const NvOpDev &dev, const LzState &st, bool beta, hipStream_t s) {
     hipLaunchKernelGGL(pro_decide_kernel, dim3(1), dim3(kDecide), 0, s, ps.d, st);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return orthog_apply(ps, dev, st, s);
+    return orthog_apply(ps, dev, st, beta, s);
 }
 
 bool pro_fusable(const ProState &ps) { return !ps.d.exact; }
 
-hipError_t pro_step_fused(ProState &ps, const NvOpDev &dev, const LzState &st, int nparts, hipStream_t s) {
-    hipLaunchKernelGGL(pro_step_kernel, dim3(1), dim3(kDecide), 0, s, ps.d, st, nparts);
+hipError_t pro_step_fused(ProState &ps, const NvOpDev &dev, const LzState &st, const double *bparts, int nparts,
+                          bool beta, hipStream_t s) {
+    hipLaunchKernelGGL(pro_step_kernel, dim3(1), dim3(kDecide), 0, s, ps.d, st, bparts, nparts);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    return orthog_apply(ps, dev, st, s);
+    return orthog_apply(ps, dev, st, beta, s);
 }
 
 // ints: [0] n, [1] cap, [2] jcap, [3] njl, [4..11] meta, then lo[cap], ro[cap], jlist[jcap];
