@@ -172,16 +172,18 @@ __device__ __forceinline__ void offdiag_accumulate2(const NvOpDev &op, const TIn
 // dig + q * M * kBlock), row q's byte offset in the vector vo[q].  SKIP
 // points the load of a step whose factor is 0 outside the buffer (it then
 // moves no memory), where a plain out-of-basis offset may land on another row.
-template <int NS, typename TIn, typename TAcc, int R, bool SKIP, int K0, int K1, int K2>
+// With S > 1 (a power of two) only every S-th term is taken, those of index
+// part modulo S.
+template <int NS, typename TIn, typename TAcc, int R, bool SKIP, int S, int K0, int K1, int K2>
 __device__ __forceinline__ void shaped_group(const NvOpDev &op, const XRes<NS, TIn> &xs, const unsigned (&vo)[R],
-                                             const uint8_t *dig, const TAcc *ftab, int tid, int g,
+                                             const uint8_t *dig, const TAcc *ftab, int tid, int g, int part,
                                              TAcc (&acc)[R][NS]) {
     constexpr int J1 = K1 ? K1 : 1, J2 = K2 ? K2 : 1;
     // all slots odd: the middle of the product is Delta = 0 (diagonal part)
     constexpr bool odd = (K0 & 1) && (K1 == 0 || (K1 & 1)) && (K2 == 0 || (K2 & 1));
     const TAcc *__restrict__ cm = cmat_of<TAcc>(op);
     const int t1 = op.tgrp[g + 1];
-    for (int t = op.tgrp[g]; t < t1; ++t) {
+    for (int t = op.tgrp[g] + ((part - op.tgrp[g]) & (S - 1)); t < t1; t += S) {
         const NvTermShape d = op.tshape[t];
         TAcc f0[R][K0], f1[R][J1], f2[R][J2];
 #pragma unroll
@@ -241,22 +243,23 @@ __device__ __forceinline__ void shaped_group(const NvOpDev &op, const XRes<NS, T
     }
 }
 
-template <int NS, typename TIn, typename TAcc, int R, bool SKIP>
+template <int NS, typename TIn, typename TAcc, int R, bool SKIP, int S = 1>
 __device__ __forceinline__ void offdiag_shaped(const NvOpDev &op, const XRes<NS, TIn> &xs, const unsigned (&vo)[R],
-                                               const uint8_t *dig, const TAcc *ftab, int tid, TAcc (&acc)[R][NS]) {
+                                               const uint8_t *dig, const TAcc *ftab, int tid, TAcc (&acc)[R][NS],
+                                               int part = 0) {
 #pragma unroll
     for (int q = 0; q < R; ++q)
 #pragma unroll
         for (int s = 0; s < NS; ++s) acc[q][s] = (TAcc)0;
-    shaped_group<NS, TIn, TAcc, R, SKIP, 2, 0, 0>(op, xs, vo, dig, ftab, tid, 0, acc);
-    shaped_group<NS, TIn, TAcc, R, SKIP, 3, 0, 0>(op, xs, vo, dig, ftab, tid, 1, acc);
-    shaped_group<NS, TIn, TAcc, R, SKIP, 4, 0, 0>(op, xs, vo, dig, ftab, tid, 2, acc);
-    shaped_group<NS, TIn, TAcc, R, SKIP, 2, 2, 0>(op, xs, vo, dig, ftab, tid, 3, acc);
-    shaped_group<NS, TIn, TAcc, R, SKIP, 3, 2, 0>(op, xs, vo, dig, ftab, tid, 4, acc);
-    shaped_group<NS, TIn, TAcc, R, SKIP, 2, 3, 0>(op, xs, vo, dig, ftab, tid, 5, acc);
-    shaped_group<NS, TIn, TAcc, R, SKIP, 1, 2, 0>(op, xs, vo, dig, ftab, tid, 6, acc);
-    shaped_group<NS, TIn, TAcc, R, SKIP, 2, 1, 0>(op, xs, vo, dig, ftab, tid, 7, acc);
-    shaped_group<NS, TIn, TAcc, R, SKIP, 2, 2, 2>(op, xs, vo, dig, ftab, tid, 8, acc);
+    shaped_group<NS, TIn, TAcc, R, SKIP, S, 2, 0, 0>(op, xs, vo, dig, ftab, tid, 0, part, acc);
+    shaped_group<NS, TIn, TAcc, R, SKIP, S, 3, 0, 0>(op, xs, vo, dig, ftab, tid, 1, part, acc);
+    shaped_group<NS, TIn, TAcc, R, SKIP, S, 4, 0, 0>(op, xs, vo, dig, ftab, tid, 2, part, acc);
+    shaped_group<NS, TIn, TAcc, R, SKIP, S, 2, 2, 0>(op, xs, vo, dig, ftab, tid, 3, part, acc);
+    shaped_group<NS, TIn, TAcc, R, SKIP, S, 3, 2, 0>(op, xs, vo, dig, ftab, tid, 4, part, acc);
+    shaped_group<NS, TIn, TAcc, R, SKIP, S, 2, 3, 0>(op, xs, vo, dig, ftab, tid, 5, part, acc);
+    shaped_group<NS, TIn, TAcc, R, SKIP, S, 1, 2, 0>(op, xs, vo, dig, ftab, tid, 6, part, acc);
+    shaped_group<NS, TIn, TAcc, R, SKIP, S, 2, 1, 0>(op, xs, vo, dig, ftab, tid, 7, part, acc);
+    shaped_group<NS, TIn, TAcc, R, SKIP, S, 2, 2, 2>(op, xs, vo, dig, ftab, tid, 8, part, acc);
 }
 
 template <typename TAcc>
@@ -454,6 +457,96 @@ __global__ __launch_bounds__(kBlock) void hv_shaped_full_kernel(NvOpDev op, cons
     diag_apply<NS>(op, r, dig, tid, v, dv);
 #pragma unroll
     for (int s = 0; s < NS; ++s) y[(size_t)s * op.D + r] = dv[s] + (double)acc[0][s];
+}
+
+// The off-diagonal rows of a workgroup whose S waves share 64 rows: every wave
+// takes each S-th term, and wave 0 gets the sum, in wave order.  For vectors
+// that leave the chip idle: with a row per thread, 72,765 rows of a cubic
+// three-state operator are 285 workgroups, about one wave a SIMD, and the
+// latency of 454 steps one after the other set the time (62 us, 41 with four
+// waves a row).
+template <int NS, typename TIn, typename TAcc, int S>
+__device__ __forceinline__ void offdiag_split(const NvOpDev &op, const XRes<NS, TIn> &xs, int r, const uint8_t *dig,
+                                              const TAcc *ftab, int lane, int wave, TAcc (&acc)[1][NS]) {
+    __shared__ TAcc part[S - 1][NS][64];
+    const unsigned vo[1] = {(unsigned)r * XRes<NS, TIn>::kEl};
+    offdiag_shaped<NS, TIn, TAcc, 1, false, S>(op, xs, vo, dig, ftab, lane, acc, wave);
+    if (wave > 0) {
+#pragma unroll
+        for (int s = 0; s < NS; ++s) part[wave - 1][s][lane] = acc[0][s];
+    }
+    __syncthreads();
+    if (wave == 0) {
+#pragma unroll
+        for (int w = 0; w < S - 1; ++w)
+#pragma unroll
+            for (int s = 0; s < NS; ++s) acc[0][s] += part[w][s][lane];
+    }
+}
+
+// hv_shaped_iter_kernel, 64 rows a workgroup of S waves that share the terms
+// (offdiag_split); a partial per workgroup.
+template <int NS, typename TIn, typename TAcc, int S>
+__global__ __launch_bounds__(64 * S) void hv_split_iter_kernel(NvOpDev op, LzState st) {
+    uint8_t *dig;
+    const TAcc *ftab = stage_tables<TAcc>(op, dig);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int b = xcd_block(blockIdx.x, gridDim.x);
+    const int64_t it = *st.iter;
+    const double *q = st.V + slot_of(it, st.nslots) * (int64_t)op.N;
+    using TX = typename std::conditional<std::is_same<TIn, F64I>::value, double, TIn>::type;
+    const XRes<NS, TIn> xs(reinterpret_cast<const TX *>(st.v64i), op.D);
+    const int r = b * 64 + lane;
+    const bool live = r < op.D;
+    if (wave == 0) {
+        if (live) digits_energy(op, r, dig, lane);
+        else for (int m = 0; m < op.M; ++m) dig[m * kBlock + lane] = 0;
+    }
+    __syncthreads();
+    TAcc acc[1][NS];
+    offdiag_split<NS, TIn, TAcc, S>(op, xs, r, dig, ftab, lane, wave, acc);
+    if (wave > 0) return;
+    TAcc *y = reinterpret_cast<TAcc *>(st.y);
+    double part = 0.0;
+    if (live) {
+        double v[NS], dv[NS];
+#pragma unroll
+        for (int s = 0; s < NS; ++s) v[s] = q[(size_t)s * op.D + r];
+        diag_apply<NS>(op, r, dig, lane, v, dv);
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            y[(size_t)s * op.D + r] = acc[0][s];
+            part += v[s] * (dv[s] + (double)acc[0][s]);
+        }
+    }
+    part = wave_sum(part);
+    if (lane == 0) st.partials[b] = part;
+}
+
+// hv_shaped_full_kernel in the same form.
+template <int NS, int S>
+__global__ __launch_bounds__(64 * S) void hv_split_full_kernel(NvOpDev op, const double *__restrict__ x,
+                                                               double *__restrict__ y) {
+    uint8_t *dig;
+    const double *ftab = stage_tables<double>(op, dig);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = xcd_block(blockIdx.x, gridDim.x) * 64 + lane;
+    const bool live = r < op.D;
+    if (wave == 0) {
+        if (live) digits_energy(op, r, dig, lane);
+        else for (int m = 0; m < op.M; ++m) dig[m * kBlock + lane] = 0;
+    }
+    __syncthreads();
+    const XRes<NS, double> xs(x, op.D);
+    double acc[1][NS];
+    offdiag_split<NS, double, double, S>(op, xs, r, dig, ftab, lane, wave, acc);
+    if (wave > 0 || !live) return;
+    double v[NS], dv[NS];
+#pragma unroll
+    for (int s = 0; s < NS; ++s) v[s] = x[(size_t)s * op.D + r];
+    diag_apply<NS>(op, r, dig, lane, v, dv);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) y[(size_t)s * op.D + r] = dv[s] + acc[0][s];
 }
 
 // ------------------------------------------------------------------------
@@ -1043,12 +1136,40 @@ static bool shaped_state_major(const NvOpDev &op) {
 
 bool hv_shaped_batch(const NvOpDev &op, int prec) { return prec == 0 ? shaped_state_major(op) : hv_shaped(op, prec); }
 
+// The FP64 H*v shares the terms of a row over the kSplitWaves waves of a
+// workgroup up to kSplitRows rows (iteration: 64 rows a partial, and no more
+// partials than the folded finishing sums take) or kSplitFullRows (standalone,
+// no partials).  33 iterations, one wave a row against four: 1,000 rows of two
+// states 539 -> 502 us, 3,500 of four states (cubic) 1349 -> 742, 72,765 of
+// three (cubic) 2467 -> 1802, 175,616 of two 1139 -> 1013, 262,144 of two
+// (cubic) 2781 -> 2528.  Two waves give less below 100,000 rows, eight lose
+// above (100,000 rows 1025 -> 943 us with four, 1010 with eight).  Standalone,
+// 460,800 rows of three states: 61.2 -> 56.6 us, cubic 298 -> 272.  Below
+// kSplitMinRows a run soon exhausts its Krylov space, after which every
+// rounding counts, and it keeps the sums of the batched kernels.
+constexpr int kSplitWaves = 4;
+constexpr int kSplitMinRows = 512;
+constexpr int kSplitRows = 64 * 4096;
+constexpr int kSplitFullRows = 1 << 19;
+static bool hv_split(const NvOpDev &op, int rows) {
+    // beside the tables, the sums of the waves after the first
+    return op.D >= kSplitMinRows && op.D <= rows &&
+           hv_lds_bytes(op, 0) + (size_t)(kSplitWaves - 1) * op.ns * 64 * sizeof(double) <= 65536;
+}
+static unsigned hv_split_blocks(const NvOpDev &op) { return (unsigned)((op.D + 63) / 64); }
+static bool hv_split_iter(const NvOpDev &op, int prec, const LzState &st) {
+    return prec == 0 && st.v64i && hv_shaped(op, prec) && !hv_shaped_skip(op, prec) && hv_split(op, kSplitRows);
+}
+
 template <int NS>
 static hipError_t hv_full_ns(const NvOpDev &op, int prec, const double *x, double *y, hipStream_t s) {
     const size_t lds = hv_lds_bytes(op, prec);
     if constexpr (NS <= kShapedMaxStates) {
         if (shaped_state_major(op)) {
-            if (prec == 0)
+            if (prec == 0 && hv_split(op, kSplitFullRows))
+                hipLaunchKernelGGL((hv_split_full_kernel<NS, kSplitWaves>), dim3(hv_split_blocks(op)),
+                                   dim3(64 * kSplitWaves), lds, s, op, x, y);
+            else if (prec == 0)
                 hipLaunchKernelGGL((hv_shaped_full_kernel<NS, double>), dim3(hv_blocks(op)), dim3(kBlock), lds, s, op,
                                    x, y);
             else
@@ -1089,7 +1210,10 @@ static hipError_t hv_iter_ns(const NvOpDev &op, int prec, const LzState &st, hip
                                        s, op, st);
                 return hipGetLastError();
             }
-            if (prec == 0)
+            if (hv_split_iter(op, prec, st))
+                hipLaunchKernelGGL((hv_split_iter_kernel<NS, F64I, double, kSplitWaves>), dim3(hv_split_blocks(op)),
+                                   dim3(64 * kSplitWaves), lds, s, op, st);
+            else if (prec == 0)
                 hipLaunchKernelGGL((hv_shaped_iter_kernel<NS, F64I, double, 1, false>), dim3(g), dim3(kBlock), lds,
                                    s, op, st);
             else
@@ -1261,7 +1385,8 @@ static hipError_t hv_iter_any(const NvOpDev &op, int prec, const LzState &st, hi
 
 int hv_iter_parts(const NvOpDev &op, int prec, const LzState &st) {
     if (fb_iter(op, prec, st)) return hv_fb_parts(op);
-    return hv2_iter(op, prec, st) ? hv2_parts(op) : hv_blocks(op);
+    if (hv2_iter(op, prec, st)) return hv2_parts(op);
+    return hv_split_iter(op, prec, st) ? (int)hv_split_blocks(op) : hv_blocks(op);
 }
 
 static hipError_t step_any(const NvOpDev &op, int prec, const LzState &st, hipStream_t s) {
