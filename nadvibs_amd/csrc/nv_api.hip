@@ -674,13 +674,7 @@ int32_t nv_hv(nv_ctx *c, int32_t prec, const double *x, double *y) {
 // Default start (shiftref = 0, Source/secondary.f90:727-783): |0> in every
 // state, weighted by statew / sum(statew), normalised.  The Franck-Condon
 // start (shiftref != 0) is built by nv::build_fc_start.
-static int32_t build_start(nv_ctx *c, double *dst) {
-    const nv::Operator &op = c->op;
-    if (op.neworigin) {
-        hipError_t e = nv::build_fc_start(op, c->dev, dst, c->stream, c->err);
-        if (e != hipSuccess) return c->err.empty() ? hip_fail(c, e, "fc start") : NV_ERR_HIP;
-        return NV_OK;
-    }
+static std::vector<double> start_values(const nv::Operator &op) {
     std::vector<double> vals(op.ns);
     // q3 = 1 at index 1 of every state; d1 = sqrt(q3.q3/nstates) = 1
     double d2 = 0.0;
@@ -693,6 +687,17 @@ static int32_t build_start(nv_ctx *c, double *dst) {
     }
     const double sc = 1.0 / std::sqrt(tot);
     for (int64_t s = 0; s < op.ns; ++s) vals[s] *= sc;
+    return vals;
+}
+
+static int32_t build_start(nv_ctx *c, double *dst) {
+    const nv::Operator &op = c->op;
+    if (op.neworigin) {
+        hipError_t e = nv::build_fc_start(op, c->dev, dst, c->stream, c->err);
+        if (e != hipSuccess) return c->err.empty() ? hip_fail(c, e, "fc start") : NV_ERR_HIP;
+        return NV_OK;
+    }
+    const std::vector<double> vals = start_values(op);
     if (!c->d_startvals) NV_HIP(c, hipMalloc(&c->d_startvals, NV_MAXS * sizeof(double)));
     NV_HIP(c, hipMemcpyAsync(c->d_startvals, vals.data(), op.ns * sizeof(double), hipMemcpyHostToDevice, c->stream));
     NV_HIP(c, nv::launch_fill_start(dst, op.D, (int)op.ns, c->d_startvals, c->stream));
@@ -2186,13 +2191,21 @@ struct nv_batch {
     int64_t *voff_d = nullptr, *loff_d = nullptr, *iter_d = nullptr;
     nv::BatchTile *tiles_d = nullptr;
     int32_t *tile0_d = nullptr;
+    nv::BatchStart *starts_d = nullptr;
+    size_t starts_cap = 0;
     std::vector<void *> allocs, run_allocs;
     size_t lds_hv = 0, lds_step = 0;
+    bool tuned = false;  // nv_batch_tune has chosen rows, tiles and form
     bool rows4 = false;  // lds_hv holds the digits of four rows per thread (FP32 shaped H*v)
     hipGraphExec_t graph = nullptr;
     hipGraphExec_t graph16 = nullptr;  // 16 iterations
     int bs = 256;
     std::vector<nv::BatchGroup> groups;
+    // alpha and beta of the first host_last iterations as one copy brought them (alpha first, [P][ld]
+    // each); -1: none
+    std::mutex host_mu;
+    std::vector<double> host_ab;
+    int64_t host_last = -1;
 };
 
 namespace {
@@ -2208,6 +2221,17 @@ int32_t bfail(nv_batch *b, int32_t code, const std::string &msg) {
         hipError_t e_ = (call);                                                                     \
         if (e_ != hipSuccess) return bfail((b), NV_ERR_HIP, std::string(#call) + ": " + hipGetErrorString(e_)); \
     } while (0)
+
+void batch_release_graphs(nv_batch *b) {
+    if (b->graph) {
+        hipGraphExecDestroy(b->graph);
+        b->graph = nullptr;
+    }
+    if (b->graph16) {
+        hipGraphExecDestroy(b->graph16);
+        b->graph16 = nullptr;
+    }
+}
 
 // Tile table for bs rows per tile: problems grouped by their number of
 // states (one specialised launch per group), each problem's tiles contiguous
@@ -2249,14 +2273,7 @@ hipError_t batch_tiles(nv_batch *b, int bs) {
     b->d.bs = bs;
     b->bs = bs;
     // captured iterations name the tiles
-    if (b->graph) {
-        hipGraphExecDestroy(b->graph);
-        b->graph = nullptr;
-    }
-    if (b->graph16) {
-        hipGraphExecDestroy(b->graph16);
-        b->graph16 = nullptr;
-    }
+    batch_release_graphs(b);
     return e;
 }
 
@@ -2271,14 +2288,7 @@ hipError_t batch_enqueue(nv_batch *b, bool absolute, int64_t it) {
 }
 
 void batch_release_run(nv_batch *b) {
-    if (b->graph) {
-        hipGraphExecDestroy(b->graph);
-        b->graph = nullptr;
-    }
-    if (b->graph16) {
-        hipGraphExecDestroy(b->graph16);
-        b->graph16 = nullptr;
-    }
+    batch_release_graphs(b);
     for (void *p : b->run_allocs) hipFree(p);
     b->run_allocs.clear();
     b->ready = false;
@@ -2359,7 +2369,7 @@ int32_t nv_batch_destroy(nv_batch *b) {
     if (b->stream) hipStreamSynchronize(b->stream);
     batch_release_run(b);
     for (void *p : {(void *)b->ops_d, (void *)b->voff_d, (void *)b->loff_d, (void *)b->iter_d, (void *)b->tiles_d,
-                    (void *)b->tile0_d})
+                    (void *)b->tile0_d, (void *)b->starts_d})
         if (p) hipFree(p);
     for (nv_ctx *c : b->ctx) nv_destroy(c);
     if (b->stream) hipStreamDestroy(b->stream);
@@ -2369,41 +2379,81 @@ int32_t nv_batch_destroy(nv_batch *b) {
 
 const char *nv_batch_last_error(const nv_batch *b) { return b ? b->err.c_str() : g_create_error.c_str(); }
 
+// A run of the shape of the one before keeps its buffers and its captured
+// iterations: releasing and allocating 440 MB and capturing 16 iterations cost
+// more than the iterations did (64 problems, 13.7M elements, 17 iterations in
+// FP32: 41 ms in all, 10 ms of them in the iterations' kernels).
 int32_t nv_batch_init(nv_batch *b, int64_t niter, int32_t prec) {
     if (!b) return NV_ERR_ARG;
     if (niter < 1) return bfail(b, NV_ERR_ARG, "niter must be >= 1");
     if (prec != NV_PREC_F64 && prec != NV_PREC_F32) return bfail(b, NV_ERR_ARG, "batch runs support F64 and F32");
     NV_BHIP(b, hipSetDevice(b->device));
     NV_BHIP(b, hipStreamSynchronize(b->stream));
-    batch_release_run(b);
-    const int64_t P = (int64_t)b->ctx.size(), ld = niter + 2;
-    int64_t maxtiles = 0;
-    for (nv_ctx *c : b->ctx) maxtiles += (c->op.D + 63) / 64;  // the smallest tile size
-    auto alloc = [&](size_t bytes, void **p) -> hipError_t {
-        hipError_t er = hipMalloc(p, bytes);
-        if (er == hipSuccess) b->run_allocs.push_back(*p);
-        return er;
-    };
-    double *V = nullptr, *al = nullptr, *be = nullptr, *parts = nullptr;
-    void *vlo = nullptr, *y = nullptr;
-    NV_BHIP(b, alloc((size_t)3 * b->Ntot * sizeof(double), (void **)&V));
-    NV_BHIP(b, alloc((size_t)b->Ntot * (prec == NV_PREC_F64 ? 8 : 4), &y));
-    if (prec == NV_PREC_F32) {
-        NV_BHIP(b, alloc((size_t)b->Ltot * sizeof(float), &vlo));
-        NV_BHIP(b, hipMemsetAsync(vlo, 0, (size_t)b->Ltot * sizeof(float), b->stream));
+    const bool same = b->ready && b->niter == niter && b->prec == prec;
+    if (!same) batch_release_run(b);
+    b->ready = false;
+    {
+        std::lock_guard<std::mutex> lock(b->host_mu);
+        b->host_last = -1;
     }
-    NV_BHIP(b, alloc((size_t)P * ld * sizeof(double), (void **)&al));
-    NV_BHIP(b, alloc((size_t)P * ld * sizeof(double), (void **)&be));
-    NV_BHIP(b, alloc((size_t)maxtiles * sizeof(double), (void **)&parts));
+    const int64_t P = (int64_t)b->ctx.size(), ld = niter + 2;
+    double *V = b->d.V, *al = b->d.alpha, *parts = b->d.partials;
+    void *vlo = b->d.vlo, *y = b->d.y;
+    if (!same) {
+        int64_t maxtiles = 0;
+        for (nv_ctx *c : b->ctx) maxtiles += (c->op.D + 63) / 64;  // the smallest tile size
+        auto alloc = [&](size_t bytes, void **p) -> hipError_t {
+            hipError_t er = hipMalloc(p, bytes);
+            if (er == hipSuccess) b->run_allocs.push_back(*p);
+            return er;
+        };
+        vlo = nullptr;
+        NV_BHIP(b, alloc((size_t)3 * b->Ntot * sizeof(double), (void **)&V));
+        NV_BHIP(b, alloc((size_t)b->Ntot * (prec == NV_PREC_F64 ? 8 : 4), &y));
+        if (prec == NV_PREC_F32) NV_BHIP(b, alloc((size_t)b->Ltot * sizeof(float), &vlo));
+        // beta behind alpha, so that one copy takes both
+        NV_BHIP(b, alloc((size_t)2 * P * ld * sizeof(double), (void **)&al));
+        NV_BHIP(b, alloc((size_t)maxtiles * sizeof(double), (void **)&parts));
+    }
+    double *be = al + P * ld;
+    // (the padding of the FP32 copy stays zero)
+    if (vlo && !same) NV_BHIP(b, hipMemsetAsync(vlo, 0, (size_t)b->Ltot * sizeof(float), b->stream));
     NV_BHIP(b, hipMemsetAsync(V, 0, (size_t)3 * b->Ntot * sizeof(double), b->stream));
-    NV_BHIP(b, hipMemsetAsync(al, 0, (size_t)P * ld * sizeof(double), b->stream));
-    NV_BHIP(b, hipMemsetAsync(be, 0, (size_t)P * ld * sizeof(double), b->stream));
-    // the start vectors below are plain copies: the clears must have landed first
-    NV_BHIP(b, hipStreamSynchronize(b->stream));
-    // start vectors (each problem's own: default or Franck-Condon) into slot 1, beta(0) = |start|
+    NV_BHIP(b, hipMemsetAsync(al, 0, (size_t)2 * P * ld * sizeof(double), b->stream));
+    // Start vectors (each problem's own) into slot 1, beta(0) = |start|.  The default ones differ
+    // from the cleared slot in a value per state, which one launch places for all problems (a start
+    // vector at a time through the host took 17 of the 41 ms); a Franck-Condon one is built by its
+    // own context.
     std::vector<double> beta0(P * ld, 0.0);
+    std::vector<nv::BatchStart> pts;
     for (int64_t p = 0; p < P; ++p) {
         nv_ctx *c = b->ctx[p];
+        if (c->op.neworigin) continue;
+        const std::vector<double> vals = start_values(c->op);
+        double nn = 0.0;
+        for (int64_t s = 0; s < c->op.ns; ++s) {
+            nn += vals[s] * vals[s];
+            pts.push_back({b->Ntot + b->voff[p] + s * c->op.D, vals[s]});
+        }
+        beta0[p * ld] = std::sqrt(nn);
+    }
+    if (pts.size() > b->starts_cap) {
+        if (b->starts_d) hipFree(b->starts_d);
+        b->starts_d = nullptr;
+        b->starts_cap = 0;
+        NV_BHIP(b, hipMalloc(&b->starts_d, pts.size() * sizeof(nv::BatchStart)));
+        b->starts_cap = pts.size();
+    }
+    if (!pts.empty()) {
+        NV_BHIP(b, hipMemcpyAsync(b->starts_d, pts.data(), pts.size() * sizeof(nv::BatchStart), hipMemcpyHostToDevice,
+                                  b->stream));
+        NV_BHIP(b, nv::launch_batch_start(b->starts_d, (int64_t)pts.size(), V, b->stream));
+    }
+    // the start vectors below are plain copies: the clears must have landed first
+    NV_BHIP(b, hipStreamSynchronize(b->stream));
+    for (int64_t p = 0; p < P; ++p) {
+        nv_ctx *c = b->ctx[p];
+        if (!c->op.neworigin) continue;
         std::vector<double> q(c->op.N);
         int32_t rc = nv_start_vector(c, q.data());
         if (rc != NV_OK) return bfail(b, rc, "problem " + std::to_string(p) + ": " + c->err);
@@ -2434,14 +2484,23 @@ int32_t nv_batch_init(nv_batch *b, int64_t niter, int32_t prec) {
     // four rows per thread (FP32, shaped form) where their digits fit in 64 KB of LDS
     b->rows4 = prec != NV_PREC_F64 && b->d.shaped[1] != 0 && lds4 <= 65536;
     if (b->rows4) b->lds_hv = lds4;
+    int rows = b->d.rows;
+    // FP32 rows per thread of the shaped form, where nv_batch_tune has not chosen: more rows share a
+    // term's descriptors and keep more loads in flight, fewer leave more waves.  17 iterations at 1,
+    // 2, 4 rows per thread: 22,400 tiles 12.9, 10.6, 9.9 ms; 3,370 tiles 2.47, 2.18, 2.16; 1,860
+    // tiles 1.65, 1.52, 1.67; 640 tiles 1.12, 1.16, 1.31.
+    if (!b->tuned && prec != NV_PREC_F64 && b->d.shaped[1])
+        rows = b->d.T >= 4096 && b->rows4 ? 4 : b->d.T >= 1024 ? 2 : 1;
     if (const char *r = std::getenv("NV_BATCH_ROWS")) {
         const int v = std::atoi(r);
         if (v != 1 && v != 2 && v != 4) return bfail(b, NV_ERR_ARG, "NV_BATCH_ROWS must be 1, 2 or 4");
         if (v > 1 && prec == NV_PREC_F64) return bfail(b, NV_ERR_ARG, "NV_BATCH_ROWS above 1 needs FP32 H*v");
         if (v == 4 && (!b->rows4 || b->bs < 256))
             return bfail(b, NV_ERR_ARG, "four rows per thread need the shaped form, 256-row tiles and LDS room");
-        b->d.rows = v;
+        rows = v;
     }
+    if (rows != b->d.rows) batch_release_graphs(b);  // captured iterations name the kernel
+    b->d.rows = rows;
     b->ready = true;
     return NV_OK;
 }
@@ -2494,11 +2553,17 @@ int32_t nv_batch_coefficients(nv_batch *b, int64_t p, double *alpha, double *bet
     if (!b->ready) return bfail(b, NV_ERR_STATE, "no batch run");
     if (p < 0 || p >= (int64_t)b->ctx.size()) return bfail(b, NV_ERR_ARG, "problem index out of range");
     NV_BHIP(b, hipSetDevice(b->device));
-    NV_BHIP(b, hipStreamSynchronize(b->stream));
-    const int64_t n = b->last;
-    if (alpha && n > 0)
-        NV_BHIP(b, hipMemcpy(alpha, b->d.alpha + p * b->d.ld + 1, n * sizeof(double), hipMemcpyDeviceToHost));
-    if (beta) NV_BHIP(b, hipMemcpy(beta, b->d.beta + p * b->d.ld, (n + 1) * sizeof(double), hipMemcpyDeviceToHost));
+    const int64_t n = b->last, all = (int64_t)b->ctx.size() * b->d.ld;
+    // two copies a problem took 1.5 ms for 64 problems
+    std::lock_guard<std::mutex> lock(b->host_mu);
+    if (b->host_last != n) {
+        NV_BHIP(b, hipStreamSynchronize(b->stream));
+        b->host_ab.resize(2 * all);
+        NV_BHIP(b, hipMemcpy(b->host_ab.data(), b->d.alpha, 2 * all * sizeof(double), hipMemcpyDeviceToHost));
+        b->host_last = n;
+    }
+    if (alpha && n > 0) std::copy_n(b->host_ab.data() + p * b->d.ld + 1, n, alpha);
+    if (beta) std::copy_n(b->host_ab.data() + all + p * b->d.ld, n + 1, beta);
     return NV_OK;
 }
 
@@ -2564,6 +2629,7 @@ int32_t nv_batch_tune(nv_batch *b, char *report, int64_t len) {
     if (e == hipSuccess) e = batch_tiles(b, best.bs);
     b->d.rows = best.rows;
     b->d.steps = best.steps;
+    b->tuned = true;
     // alpha(1) of the timing launches is recomputed by the first iteration
     if (e == hipSuccess) e = hipMemsetAsync(b->d.alpha, 0, (size_t)b->ctx.size() * b->d.ld * sizeof(double), b->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(b->stream);

@@ -1546,6 +1546,11 @@ __device__ __forceinline__ void batch_hv_row(const NvOpDev &op, const TIn *x, co
     }
 }
 
+__global__ __launch_bounds__(kBlock) void batch_start_kernel(const BatchStart *pts, int64_t n, double *v) {
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) v[pts[i].at] = pts[i].value;
+}
+
 template <typename TIn>
 __global__ __launch_bounds__(kBlock) void batch_normalize_kernel(BatchDev b) {
     const BatchTile tl = b.tiles[blockIdx.x];
@@ -1742,6 +1747,11 @@ __global__ __launch_bounds__(256) void batch_finish_kernel(BatchDev b, double *d
         const int64_t it = *b.iter;
         dst[(int64_t)p * b.ld + it] = take_sqrt ? sqrt(s) : s;
     }
+}
+
+hipError_t launch_batch_start(const BatchStart *pts, int64_t n, double *v, hipStream_t s) {
+    hipLaunchKernelGGL(batch_start_kernel, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, pts, n, v);
+    return hipGetLastError();
 }
 
 size_t batch_hv_lds(const NvOpDev &op, int prec) { return hv_lds_bytes(op, prec); }

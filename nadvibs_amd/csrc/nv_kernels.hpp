@@ -208,6 +208,12 @@ struct BatchDev {
 struct BatchGroup {
     int ns, t0, nt;
 };
+// v[at] = value for the nonzero elements of the default start vectors.
+struct BatchStart {
+    int64_t at;
+    double value;
+};
+hipError_t launch_batch_start(const BatchStart *pts, int64_t n, double *v, hipStream_t s);
 size_t batch_hv_lds(const NvOpDev &op, int prec);
 // update_lanczos, Hv (+ alpha finish) and lanczos_step (+ beta finish) for every problem.
 hipError_t launch_batch_normalize(const BatchDev &b, int prec, hipStream_t s);
