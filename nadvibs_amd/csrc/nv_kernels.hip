@@ -495,7 +495,9 @@ __global__ __launch_bounds__(64 * S) void hv_split_iter_kernel(NvOpDev op, LzSta
     const int64_t it = *st.iter;
     const double *q = st.V + slot_of(it, st.nslots) * (int64_t)op.N;
     using TX = typename std::conditional<std::is_same<TIn, F64I>::value, double, TIn>::type;
-    const XRes<NS, TIn> xs(reinterpret_cast<const TX *>(st.v64i), op.D);
+    const TX *x = std::is_same<TIn, F64I>::value ? reinterpret_cast<const TX *>(st.v64i)
+                                                 : reinterpret_cast<const TX *>(st.vlo);
+    const XRes<NS, TIn> xs(x, op.D);
     const int r = b * 64 + lane;
     const bool live = r < op.D;
     if (wave == 0) {
@@ -524,11 +526,11 @@ __global__ __launch_bounds__(64 * S) void hv_split_iter_kernel(NvOpDev op, LzSta
 }
 
 // hv_shaped_full_kernel in the same form.
-template <int NS, int S>
+template <int NS, typename TAcc, int S>
 __global__ __launch_bounds__(64 * S) void hv_split_full_kernel(NvOpDev op, const double *__restrict__ x,
                                                                double *__restrict__ y) {
     uint8_t *dig;
-    const double *ftab = stage_tables<double>(op, dig);
+    const TAcc *ftab = stage_tables<TAcc>(op, dig);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = xcd_block(blockIdx.x, gridDim.x) * 64 + lane;
     const bool live = r < op.D;
@@ -538,15 +540,15 @@ __global__ __launch_bounds__(64 * S) void hv_split_full_kernel(NvOpDev op, const
     }
     __syncthreads();
     const XRes<NS, double> xs(x, op.D);
-    double acc[1][NS];
-    offdiag_split<NS, double, double, S>(op, xs, r, dig, ftab, lane, wave, acc);
+    TAcc acc[1][NS];
+    offdiag_split<NS, double, TAcc, S>(op, xs, r, dig, ftab, lane, wave, acc);
     if (wave > 0 || !live) return;
     double v[NS], dv[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) v[s] = x[(size_t)s * op.D + r];
     diag_apply<NS>(op, r, dig, lane, v, dv);
 #pragma unroll
-    for (int s = 0; s < NS; ++s) y[(size_t)s * op.D + r] = dv[s] + acc[0][s];
+    for (int s = 0; s < NS; ++s) y[(size_t)s * op.D + r] = dv[s] + (double)acc[0][s];
 }
 
 // ------------------------------------------------------------------------
@@ -1147,18 +1149,26 @@ bool hv_shaped_batch(const NvOpDev &op, int prec) { return prec == 0 ? shaped_st
 // 460,800 rows of three states: 61.2 -> 56.6 us, cubic 298 -> 272.  Below
 // kSplitMinRows a run soon exhausts its Krylov space, after which every
 // rounding counts, and it keeps the sums of the batched kernels.
+// In FP32 it serves operators of kSplitTerms32 terms or more: those whose
+// steps are too many for the run-time compiled kernel.  17 iterations, cubic
+// operators of 9 and 10 modes: 1,536 rows of four states 2061 -> 720 us,
+// 19,683 of two 1478 -> 646, 104,976 of three 2281 -> 1860, 248,832 of three
+// 4093 -> 3793; the error against 64 bits falls by a third (four short FP32
+// sums instead of one long one).
 constexpr int kSplitWaves = 4;
+constexpr int kSplitTerms32 = 200;
 constexpr int kSplitMinRows = 512;
 constexpr int kSplitRows = 64 * 4096;
 constexpr int kSplitFullRows = 1 << 19;
-static bool hv_split(const NvOpDev &op, int rows) {
+static bool hv_split(const NvOpDev &op, int prec, int rows) {
     // beside the tables, the sums of the waves after the first
-    return op.D >= kSplitMinRows && op.D <= rows &&
+    return (prec == 0 || (prec == 1 && op.nterms >= kSplitTerms32)) && op.D >= kSplitMinRows && op.D <= rows &&
            hv_lds_bytes(op, 0) + (size_t)(kSplitWaves - 1) * op.ns * 64 * sizeof(double) <= 65536;
 }
 static unsigned hv_split_blocks(const NvOpDev &op) { return (unsigned)((op.D + 63) / 64); }
 static bool hv_split_iter(const NvOpDev &op, int prec, const LzState &st) {
-    return prec == 0 && st.v64i && hv_shaped(op, prec) && !hv_shaped_skip(op, prec) && hv_split(op, kSplitRows);
+    return (prec == 0 ? (void *)st.v64i : st.vlo) && hv_shaped(op, prec) && !hv_shaped_skip(op, prec) &&
+           hv_split(op, prec, kSplitRows);
 }
 
 template <int NS>
@@ -1166,8 +1176,11 @@ static hipError_t hv_full_ns(const NvOpDev &op, int prec, const double *x, doubl
     const size_t lds = hv_lds_bytes(op, prec);
     if constexpr (NS <= kShapedMaxStates) {
         if (shaped_state_major(op)) {
-            if (prec == 0 && hv_split(op, kSplitFullRows))
-                hipLaunchKernelGGL((hv_split_full_kernel<NS, kSplitWaves>), dim3(hv_split_blocks(op)),
+            if (prec == 0 && hv_split(op, prec, kSplitFullRows))
+                hipLaunchKernelGGL((hv_split_full_kernel<NS, double, kSplitWaves>), dim3(hv_split_blocks(op)),
+                                   dim3(64 * kSplitWaves), lds, s, op, x, y);
+            else if (hv_split(op, prec, kSplitFullRows))
+                hipLaunchKernelGGL((hv_split_full_kernel<NS, float, kSplitWaves>), dim3(hv_split_blocks(op)),
                                    dim3(64 * kSplitWaves), lds, s, op, x, y);
             else if (prec == 0)
                 hipLaunchKernelGGL((hv_shaped_full_kernel<NS, double>), dim3(hv_blocks(op)), dim3(kBlock), lds, s, op,
@@ -1210,8 +1223,12 @@ static hipError_t hv_iter_ns(const NvOpDev &op, int prec, const LzState &st, hip
                                        s, op, st);
                 return hipGetLastError();
             }
-            if (hv_split_iter(op, prec, st))
+            const bool split = hv_split_iter(op, prec, st);
+            if (split && prec == 0)
                 hipLaunchKernelGGL((hv_split_iter_kernel<NS, F64I, double, kSplitWaves>), dim3(hv_split_blocks(op)),
+                                   dim3(64 * kSplitWaves), lds, s, op, st);
+            else if (split)
+                hipLaunchKernelGGL((hv_split_iter_kernel<NS, float, float, kSplitWaves>), dim3(hv_split_blocks(op)),
                                    dim3(64 * kSplitWaves), lds, s, op, st);
             else if (prec == 0)
                 hipLaunchKernelGGL((hv_shaped_iter_kernel<NS, F64I, double, 1, false>), dim3(g), dim3(kBlock), lds,

@@ -1,8 +1,8 @@
-"""GPU: FP64 H*v with the terms of a row shared over the waves of a workgroup,
+"""GPU: H*v with the terms of a row shared over the waves of a workgroup,
 against the step-table kernels, which the oracle holds: ragged and full last
-workgroups, fewer terms than waves, one to ten states,
-every order, states coupled through the diagonal part, and the row counts on
-both sides of the lines between which the terms are shared."""
+workgroups, fewer terms than waves, one to ten states, every order, states
+coupled through the diagonal part, and the row counts on both sides of the lines
+between which the terms are shared; FP32 with the many terms that it takes there."""
 import numpy as np
 import pytest
 
@@ -22,7 +22,9 @@ CASES = [
     (10, [13, 8, 5], 2, 5.0, 3),
     (3, [11, 9, 7, 5], 3, 30.0, 3),
     (1, [64, 64, 64], 2, 0.0, 3),
+    (1, [64, 17, 241], 2, 0.0, 3),
     (1, [61, 63, 69], 2, 0.0, 3),
+    (2, [64, 64, 128], 3, 10.0, 3),
     (1, [74, 85, 84], 2, 0.0, 3),
 ]
 
@@ -53,3 +55,41 @@ def test_shared_terms_match_the_step_tables(case, monkeypatch):
         assert np.max(np.abs(y - ref)) <= 1e-13 * np.max(np.abs(ref))
         for got, want in zip(ab, coefficients(eng)):
             assert np.max(np.abs(got - want)) <= 1e-11 * np.max(np.abs(want))
+
+
+# cubic operators of 219 and 285 terms
+MANY = [
+    (2, [2] * 9, 0.0, 3),
+    (4, [2] * 9 + [3], 10.0, 3),
+    (3, [3] * 9, 5.0, 0),
+    (1, [5, 4] + [3] * 7, 0.0, 3),
+    (2, [4] * 4 + [2] * 10, 0.0, 3),
+]
+
+
+@pytest.mark.parametrize("case", MANY, ids=lambda c: f"{c[0]}x{'-'.join(map(str, c[1]))}")
+def test_shared_terms_fp32(case, monkeypatch):
+    """Bounds: a row sums at most about 2,000 products in FP32, within 2e-6 of the largest element,
+    and the coefficients of 12 steps within 5e-6, against FP64 step tables."""
+    for v in ("NV_HV_KERNEL", "NV_HV_FB"):
+        monkeypatch.delenv(v, raising=False)
+    ns, nf, offe, quirks = case
+    p = make_problem(ns, nf, 3, (400, 2500), 200.0, 60.0, 40.0, cubic=10.0, seed=len(nf), quirks=quirks,
+                     offdiag_even=offe)
+    print(f"case {case} n={p.n}", flush=True)
+    x = np.random.default_rng(3).standard_normal(p.n)
+
+    def results(eng, prec):
+        y = eng.hv(x, prec)
+        eng.lanczos_init(niter=12, reorthog=0, prec=prec)
+        eng.run(1, 12)
+        a, b, _ = eng.coefficients()
+        return y, np.array(a), np.array(b)
+
+    with Engine(p) as eng:
+        eng.select_hv_kernel("steps")
+        ref = results(eng, "f64")
+        eng.select_hv_kernel(True)
+        got = results(eng, "f32")
+    for tol, g, r in zip((2e-6, 5e-6, 5e-6), got, ref):
+        assert np.max(np.abs(g - r)) <= tol * np.max(np.abs(r))
