@@ -57,6 +57,7 @@ struct nv_ctx {
     std::string jit_log;
     float *hx32 = nullptr;
     void *yt[2] = {nullptr, nullptr};     // slab pass of a standalone fast-block H*v, FP64 and FP32 (in allocs)
+    bool yt_asked[2] = {false, false};    // its memory was asked for (once: a later call may be captured)
     double *hx64i = nullptr;              // interleaved FP64 copy of a standalone H*v input (two-pass form)
     void *z2 = nullptr;                   // channel scratch of the two-pass H*v
     size_t z2_bytes = 0;
@@ -604,8 +605,10 @@ static hipError_t hv_apply(nv_ctx *c, int32_t prec, const double *x, double *y, 
         const void *xin = nullptr;
         hipError_t e = interleaved_input(c, prec, x, &xin, s);
         if (e != hipSuccess) return e;
-        void *&yt = c->yt[prec == NV_PREC_F32];
-        if (!yt) yt = alloc_slab(c, prec, c->allocs);
+        const int k32 = prec == NV_PREC_F32;
+        void *&yt = c->yt[k32];
+        if (!c->yt_asked[k32]) yt = alloc_slab(c, prec, c->allocs);
+        c->yt_asked[k32] = true;
         return nv::launch_hv_fb_full(c->dev, prec, x, xin, yt, y, s);
     }
     if (use_hv2(c, prec)) {
