@@ -289,11 +289,17 @@ template <int NS> struct XRes<NS, F64I> {
 
 // One interleaved row of K values (the H*v input copies), aligned for one
 // wide store where its size allows.
-__host__ __device__ constexpr size_t il_align(size_t b) { return b % 16 == 0 ? 16 : b % 8 == 0 ? 8 : 4; }
+__host__ __device__ constexpr size_t il_align(size_t b) {
+    return b % 16 == 0 ? 16 : b % 8 == 0 ? 8 : b % 4 == 0 ? 4 : 2;
+}
 template <typename T, int K> struct alignas(il_align(sizeof(T) * K) < alignof(T) ? alignof(T)
                                                                                   : il_align(sizeof(T) * K)) IlRow {
     T v[K];
 };
+// rows follow each other without a gap, as H*v reads them (three BF16 values are 6 bytes)
+static_assert(sizeof(IlRow<__hip_bfloat16, 1>) == 2 && sizeof(IlRow<__hip_bfloat16, 3>) == 6 &&
+                  sizeof(IlRow<float, 3>) == 12 && sizeof(IlRow<double, 3>) == 24,
+              "an interleaved row holds its values and nothing else");
 
 __device__ __forceinline__ int64_t slot_of(int64_t i, int64_t nslots) { return i % nslots; }
 
