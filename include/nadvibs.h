@@ -204,7 +204,10 @@ int32_t nv_get_lanczos_vector(nv_ctx *ctx, int64_t j, double *q);
 /* Eigenvalues (ascending) of the n x n tridiagonal T with diagonal
  * alpha[0..n-1] and off-diagonal beta[1..n-1] (beta[0] = beta(0) unused),
  * intensities inten[i] = v(1,i)^2, convergence bji[i] = |beta[n] * v(n,i)|
- * and sign[i] = sign of v(1,i).  Runs on the context's device. */
+ * and sign[i] = sign of v(1,i).  Runs on the context's device.  The device
+ * workspace (40 n^2 bytes) is kept for the next solve, up to 512 MB in all for
+ * the contexts of a device; it goes back with the last of them, and when an
+ * eigensolve finds the memory short. */
 int32_t nv_ritz(nv_ctx *ctx, int64_t n, const double *alpha,
                 const double *beta, double *eval, double *inten, double *bji,
                 int32_t *sign);

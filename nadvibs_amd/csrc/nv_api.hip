@@ -19,6 +19,7 @@
 #include "nv_kernels.hpp"
 #include "nv_operator.hpp"
 #include "nv_pro.hpp"
+#include "nv_workspace.hpp"
 
 struct nv_ctx {
     int device = 0;
@@ -80,10 +81,6 @@ struct nv_ctx {
     std::vector<std::pair<hipEvent_t, hipEvent_t>> ev;
     size_t ev_used = 0;
     size_t lz_bytes_key = 0;
-
-    // device workspace of the tridiagonal eigensolve, kept between calls up to kTriKeepBytes
-    void *tri = nullptr;
-    size_t tri_bytes = 0;
 };
 
 static std::string g_create_error;
@@ -116,6 +113,73 @@ static double *scratch_of(int device) {
     std::lock_guard<std::mutex> lock(g_scratch_mutex);
     return g_scratch_ptr[device];
 }
+
+// ---- what the contexts of a device share -------------------------------------
+// The workspace of the tridiagonal eigensolve (5 n^2 doubles, 360 MB at n = 3000) is kept between
+// calls up to kTriKeepBytes a device, not a context: the problems of a batch solve one after the
+// other, each through its own context.  It goes back with the device's last context.
+constexpr size_t kTriKeepBytes = (size_t)512 << 20;
+
+struct HipAlloc {
+    static int get(void **p, size_t bytes) {
+        const hipError_t e = hipMalloc(p, bytes);
+        if (e != hipSuccess) (void)hipGetLastError();
+        return (int)e;
+    }
+    static void put(void *p) { (void)hipFree(p); }
+};
+using TriPool = nv::BlockPool<HipAlloc>;
+
+struct DeviceShared {
+    TriPool tri{kTriKeepBytes};
+    int contexts = 0;
+};
+static std::mutex g_shared_mutex;
+
+// (never destroyed: the runtime may be gone before static objects are)
+static DeviceShared &shared_of(int device) {
+    static auto *all = new std::map<int, DeviceShared>;
+    return (*all)[device];
+}
+
+static TriPool &tri_pool(int device) {
+    std::lock_guard<std::mutex> lock(g_shared_mutex);
+    return shared_of(device).tri;
+}
+
+static void context_created(int device) {
+    std::lock_guard<std::mutex> lock(g_shared_mutex);
+    ++shared_of(device).contexts;
+}
+
+static void context_destroyed(int device) {
+    std::lock_guard<std::mutex> lock(g_shared_mutex);
+    DeviceShared &d = shared_of(device);
+    if (--d.contexts == 0) d.tri.trim();
+}
+
+// A block of the eigensolve's workspace, given back once the stream is through with it.
+struct TriBlock {
+    TriPool *pool = nullptr;
+    hipStream_t stream = nullptr;
+    TriPool::Block b;
+    TriBlock() = default;
+    TriBlock(const TriBlock &) = delete;
+    TriBlock &operator=(const TriBlock &) = delete;
+    ~TriBlock() { reset(); }
+    hipError_t take(const nv_ctx *c, size_t bytes) {
+        reset();
+        pool = &tri_pool(c->device);
+        stream = c->stream;
+        return (hipError_t)pool->take(bytes, &b);
+    }
+    void reset() {
+        if (!b.p) return;
+        (void)hipStreamSynchronize(stream);
+        pool->give(b);
+        b = {};
+    }
+};
 
 namespace {
 
@@ -439,6 +503,7 @@ int32_t nv_create(const nv_problem *prob, int32_t device, nv_ctx **out) {
         return fail(nullptr, NV_ERR_ARG,
                     "factor table and mode digits exceed the 64 KiB LDS budget of the H*v kernel");
     }
+    context_created(device);
     *out = c;
     return NV_OK;
 }
@@ -456,8 +521,8 @@ int32_t nv_destroy(nv_ctx *c) {
     if (c->d_startvals) hipFree(c->d_startvals);
     if (c->hx) hipFree(c->hx);
     if (c->hy) hipFree(c->hy);
-    if (c->tri) hipFree(c->tri);
     if (c->stream) hipStreamDestroy(c->stream);
+    context_destroyed(c->device);
     delete c;
     return NV_OK;
 }
@@ -1237,36 +1302,11 @@ int32_t nv_get_lanczos_vector(nv_ctx *c, int64_t j, double *q) {
 }
 
 // ---- tridiagonal eigensolve ---------------------------------------------
-// The workspace of one eigensolve (5 n^2 doubles, 360 MB at n = 3000) stays with the context, as a
-// program solves again and again while it iterates; a larger one goes back after each call.
-constexpr size_t kTriKeepBytes = (size_t)512 << 20;
-
-static hipError_t tri_reserve(nv_ctx *c, size_t bytes) {
-    if (c->tri_bytes >= bytes) return hipSuccess;
-    if (c->tri) hipFree(c->tri);
-    c->tri = nullptr;
-    c->tri_bytes = 0;
-    hipError_t e = hipMalloc(&c->tri, bytes);
-    if (e == hipSuccess) c->tri_bytes = bytes;
-    else c->tri = nullptr;
-    return e;
-}
-
-// After the last use of an eigensolve's vectors (the stream synchronised).
-static void tri_trim(nv_ctx *c) {
-    if (c->tri_bytes <= kTriKeepBytes) return;
-    hipFree(c->tri);
-    c->tri = nullptr;
-    c->tri_bytes = 0;
-}
-
 // Eigenvalues (ascending) and eigenvectors of the tridiagonal T(alpha,
-// beta(1:n-1)) on the device.  *vec_dev (n*n doubles, vec[j*n + i] =
-// component j of root i) lies in the context's workspace until the next
-// solve; the caller ends with tri_trim.
+// beta(1:n-1)) on the device.  vecs holds the eigenvectors (n*n doubles,
+// vec[j*n + i] = component j of root i) as long as the caller keeps it.
 static int32_t tridiag_solve(nv_ctx *c, int64_t n, const double *alpha, const double *beta,
-                             std::vector<double> &root, double **vec_dev) {
-    *vec_dev = nullptr;
+                             std::vector<double> &root, TriBlock &vecs) {
     for (int64_t i = 0; i < n; ++i)
         if (!std::isfinite(alpha[i]) || !std::isfinite(beta[i + 1]))
             return fail(c, NV_ERR_ARG, "alpha/beta hold a non-finite value at iteration " + std::to_string(i + 1));
@@ -1280,8 +1320,8 @@ static int32_t tridiag_solve(nv_ctx *c, int64_t n, const double *alpha, const do
         if (i > 0) factor = std::fmax(factor, std::fabs(beta[i]));
     }
     if (n == 1 || factor == 0.0) {
-        NV_HIP(c, tri_reserve(c, (size_t)n * n * sizeof(double)));
-        double *vec = (double *)c->tri;
+        NV_HIP(c, vecs.take(c, (size_t)n * n * sizeof(double)));
+        double *vec = (double *)vecs.b.p;
         std::vector<double> eye((size_t)n * n, 0.0);
         for (int64_t i = 0; i < n; ++i) {
             eye[(size_t)i * n + i] = 1.0;
@@ -1289,7 +1329,6 @@ static int32_t tridiag_solve(nv_ctx *c, int64_t n, const double *alpha, const do
         }
         hipError_t er = hipMemcpy(vec, eye.data(), (size_t)n * n * sizeof(double), hipMemcpyHostToDevice);
         if (er != hipSuccess) return hip_fail(c, er, "tridiagonal eigenvectors");
-        *vec_dev = vec;
         return NV_OK;
     }
     double anorm = 0.0;
@@ -1313,13 +1352,15 @@ static int32_t tridiag_solve(nv_ctx *c, int64_t n, const double *alpha, const do
         at += (bytes + 255) & ~(size_t)255;
         return o;
     };
-    const size_t o_vec = carve((size_t)n * n * 8), o_lu = carve((size_t)4 * n * n * 8), o_up = carve(up.size() * 8),
-                 o_root = carve(n * 8), o_rank = carve(n * 8), o_ia = carve(n * 4),
-                 o_cnt = carve((size_t)nv::tri_grid_points(n) * 4);
-    NV_HIP(c, tri_reserve(c, at));
-    char *base = (char *)c->tri;
+    const size_t o_lu = carve((size_t)4 * n * n * 8), o_up = carve(up.size() * 8), o_root = carve(n * 8),
+                 o_rank = carve(n * 8), o_ia = carve(n * 4), o_cnt = carve((size_t)nv::tri_grid_points(n) * 4);
+    // (the factors go back before the caller allocates for what it does with the vectors)
+    TriBlock work;
+    NV_HIP(c, work.take(c, at));
+    NV_HIP(c, vecs.take(c, (size_t)n * n * sizeof(double)));
+    char *base = (char *)work.b.p;
     nv::TriWork w;
-    w.vec = (double *)(base + o_vec);
+    w.vec = (double *)vecs.b.p;
     w.lu = (double *)(base + o_lu);
     w.de = (double *)(base + o_up);
     w.d = w.de + nde;
@@ -1334,7 +1375,6 @@ static int32_t tridiag_solve(nv_ctx *c, int64_t n, const double *alpha, const do
     if (er == hipSuccess) er = hipStreamSynchronize(c->stream);
     if (er != hipSuccess) return hip_fail(c, er, "tridiagonal eigensolve");
     for (int64_t i = 0; i < n; ++i) root[i] *= anorm;
-    *vec_dev = w.vec;
     return NV_OK;
 }
 
@@ -1343,13 +1383,13 @@ int32_t nv_ritz(nv_ctx *c, int64_t n, const double *alpha, const double *beta, d
     if (!c) return NV_ERR_ARG;
     if (n < 1 || !alpha || !beta || !eval) return fail(c, NV_ERR_ARG, "bad tridiagonal arguments");
     std::vector<double> root, v1(n), vn(n);
-    double *vec = nullptr;
-    int32_t rc = tridiag_solve(c, n, alpha, beta, root, &vec);
+    TriBlock vecs;
+    int32_t rc = tridiag_solve(c, n, alpha, beta, root, vecs);
     if (rc != NV_OK) return rc;
+    const double *vec = (const double *)vecs.b.p;
     hipError_t er = hipMemcpyAsync(v1.data(), vec, n * 8, hipMemcpyDeviceToHost, c->stream);
     if (er == hipSuccess) er = hipMemcpyAsync(vn.data(), vec + (n - 1) * n, n * 8, hipMemcpyDeviceToHost, c->stream);
     if (er == hipSuccess) er = hipStreamSynchronize(c->stream);
-    tri_trim(c);
     if (er != hipSuccess) return hip_fail(c, er, "tridiagonal eigenvectors");
     const double bn = beta[n];
     for (int64_t i = 0; i < n; ++i) {
@@ -1379,9 +1419,10 @@ int32_t nv_identify_roots(nv_ctx *c, int64_t n, const double *alpha, const doubl
     if (idroots > 0 && (!top_index || !top_state || !top_phase || !top_mag2))
         return fail(c, NV_ERR_ARG, "top_* outputs missing");
     std::vector<double> root;
-    double *vec = nullptr;
-    int32_t rc = tridiag_solve(c, n, alpha, beta, root, &vec);
+    TriBlock vecs;
+    int32_t rc = tridiag_solve(c, n, alpha, beta, root, vecs);
     if (rc != NV_OK) return rc;
+    const double *vec = (const double *)vecs.b.p;
     std::vector<void *> tmp;
     auto alloc = [&](size_t bytes, void **p) -> hipError_t {
         hipError_t er = hipMalloc(p, bytes);
@@ -1428,7 +1469,6 @@ int32_t nv_identify_roots(nv_ctx *c, int64_t n, const double *alpha, const doubl
         er = hipMemcpyAsync(vectors, Y, (size_t)nroots * N * 8, hipMemcpyDeviceToHost, c->stream);
     if (er == hipSuccess) er = hipStreamSynchronize(c->stream);
     for (void *p : tmp) hipFree(p);
-    tri_trim(c);
     if (er != hipSuccess) return hip_fail(c, er, "identify_roots");
     // intensities relative to the strongest of the nroots roots (Source/top.f90:1165-1168)
     double intfactor = 0.0;
@@ -1784,9 +1824,10 @@ static int32_t spectrum_common(nv_ctx *c, int64_t n, const double *alpha, const 
     if (n < 1 || ng < 1 || !alpha || !beta || !grid || !(sigma > 0) || (origin != 0 && origin != 1))
         return fail(c, NV_ERR_ARG, "bad spectrum arguments");
     std::vector<double> root;
-    double *vec = nullptr;
-    int32_t rc = tridiag_solve(c, n, alpha, beta, root, &vec);
+    TriBlock vecs;
+    int32_t rc = tridiag_solve(c, n, alpha, beta, root, vecs);
     if (rc != NV_OK) return rc;
+    const double *vec = (const double *)vecs.b.p;
     std::vector<void *> tmp;
     auto alloc = [&](size_t bytes, void **p) -> hipError_t {
         hipError_t er = hipMalloc(p, bytes);
@@ -1822,7 +1863,6 @@ static int32_t spectrum_common(nv_ctx *c, int64_t n, const double *alpha, const 
     }
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     for (void *p : tmp) hipFree(p);
-    tri_trim(c);
     if (e != hipSuccess) return hip_fail(c, e, "spectrum");
     return NV_OK;
 }
