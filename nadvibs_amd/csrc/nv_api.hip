@@ -158,6 +158,26 @@ static void context_destroyed(int device) {
     if (--d.contexts == 0) d.tri.trim();
 }
 
+// hipMalloc that takes back what lies idle when the memory is short.  A failure leaves no error
+// behind for the launches after it to report.
+hipError_t nv::device_alloc(void **p, size_t bytes) {
+    hipError_t e = (hipError_t)HipAlloc::get(p, bytes);
+    int device = 0;
+    if (e == hipErrorOutOfMemory && hipGetDevice(&device) == hipSuccess && tri_pool(device).trim())
+        e = (hipError_t)HipAlloc::get(p, bytes);
+    if (e != hipSuccess) *p = nullptr;
+    return e;
+}
+
+static bool drop_slab(nv_ctx *c);
+
+// The same for a call on context c, which can also do without the slab buffer of its run.
+static hipError_t ctx_alloc(nv_ctx *c, void **p, size_t bytes) {
+    hipError_t e = nv::device_alloc(p, bytes);
+    if (e == hipErrorOutOfMemory && drop_slab(c)) e = nv::device_alloc(p, bytes);
+    return e;
+}
+
 // A block of the eigensolve's workspace, given back once the stream is through with it.
 struct TriBlock {
     TriPool *pool = nullptr;
@@ -167,11 +187,13 @@ struct TriBlock {
     TriBlock(const TriBlock &) = delete;
     TriBlock &operator=(const TriBlock &) = delete;
     ~TriBlock() { reset(); }
-    hipError_t take(const nv_ctx *c, size_t bytes) {
+    hipError_t take(nv_ctx *c, size_t bytes) {
         reset();
         pool = &tri_pool(c->device);
         stream = c->stream;
-        return (hipError_t)pool->take(bytes, &b);
+        hipError_t e = (hipError_t)pool->take(bytes, &b);
+        if (e == hipErrorOutOfMemory && drop_slab(c)) e = (hipError_t)pool->take(bytes, &b);
+        return e;
     }
     void reset() {
         if (!b.p) return;
@@ -204,7 +226,7 @@ hipError_t upload(nv_ctx *c, const std::vector<T> &h, const T **out, std::vector
     *out = nullptr;
     if (h.empty()) return hipSuccess;
     void *p = nullptr;
-    hipError_t e = hipMalloc(&p, h.size() * sizeof(T));
+    hipError_t e = ctx_alloc(c, &p, h.size() * sizeof(T));
     if (e != hipSuccess) return e;
     list.push_back(p);
     e = hipMemcpy(p, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice);
@@ -236,6 +258,19 @@ void release_lanczos(nv_ctx *c) {
 bool valid_prec(int32_t p) { return p == NV_PREC_F64 || p == NV_PREC_F32 || p == NV_PREC_BF16; }
 
 }  // namespace
+
+// Frees the slab buffer of the run, whose iterations then take every step in the sweep; whether
+// there was one to free.  Not where segments are recomputed from checkpoints: the recomputation is
+// checked bit for bit, and the two forms add in different orders.
+static bool drop_slab(nv_ctx *c) {
+    if (!c->st.yt || c->cp) return false;
+    if (hipStreamSynchronize(c->stream) != hipSuccess) return false;
+    release_graphs(c);  // captured iterations name it
+    c->lz_allocs.erase(std::find(c->lz_allocs.begin(), c->lz_allocs.end(), c->st.yt));
+    (void)hipFree(c->st.yt);
+    c->st.yt = nullptr;
+    return true;
+}
 
 extern "C" {
 
@@ -481,7 +516,7 @@ int32_t nv_create(const nv_problem *prob, int32_t device, nv_ctx **out) {
         }
     if (e == hipSuccess) {
         void *p = nullptr;
-        e = hipMalloc(&p, (size_t)op.N * sizeof(double));
+        e = ctx_alloc(c, &p, (size_t)op.N * sizeof(double));
         if (e == hipSuccess) {
             c->allocs.push_back(p);
             d.dg = (const double *)p;
@@ -594,7 +629,7 @@ static hipError_t ensure_z2(nv_ctx *c, size_t bytes) {
     if (c->z2) hipFree(c->z2);
     c->z2 = nullptr;
     c->z2_bytes = 0;
-    e = hipMalloc(&c->z2, bytes);
+    e = ctx_alloc(c, &c->z2, bytes);
     if (e == hipSuccess) c->z2_bytes = bytes;
     else c->z2 = nullptr;
     return e;
@@ -611,7 +646,7 @@ static hipError_t alloc_interleaved(nv_ctx *c, size_t el, std::vector<void *> &o
     const size_t nsp = (size_t)nv_lo_stride((int)c->op.ns), pad = il_pad(c);
     const size_t bytes = ((size_t)c->op.D + 2 * pad) * nsp * el;
     void *p = nullptr;
-    hipError_t e = hipMalloc(&p, bytes);
+    hipError_t e = ctx_alloc(c, &p, bytes);
     if (e != hipSuccess) return e;
     owner.push_back(p);
     e = hipMemsetAsync(p, 0, bytes, s);
@@ -656,10 +691,7 @@ static void *alloc_slab(nv_ctx *c, int32_t prec, std::vector<void *> &owner) {
     const size_t bytes = nv::hv_slab_bytes(c->dev, prec);
     void *p = nullptr;
     if (bytes == 0) return nullptr;
-    if (hipMalloc(&p, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
+    if (nv::device_alloc(&p, bytes) != hipSuccess) return nullptr;
     owner.push_back(p);
     return p;
 }
@@ -727,8 +759,8 @@ int32_t nv_hv(nv_ctx *c, int32_t prec, const double *x, double *y) {
     NV_HIP(c, hipSetDevice(c->device));
     const size_t bytes = (size_t)c->op.N * sizeof(double);
     if (!c->hx) {
-        NV_HIP(c, hipMalloc(&c->hx, bytes));
-        NV_HIP(c, hipMalloc(&c->hy, bytes));
+        NV_HIP(c, ctx_alloc(c, (void **)&c->hx, bytes));
+        NV_HIP(c, ctx_alloc(c, (void **)&c->hy, bytes));
     }
     NV_HIP(c, hipMemcpyAsync(c->hx, x, bytes, hipMemcpyHostToDevice, c->stream));
     int32_t rc = nv_hv_device(c, prec, c->hx, c->hy, c->stream);
@@ -766,7 +798,7 @@ static int32_t build_start(nv_ctx *c, double *dst) {
         return NV_OK;
     }
     const std::vector<double> vals = start_values(op);
-    if (!c->d_startvals) NV_HIP(c, hipMalloc(&c->d_startvals, NV_MAXS * sizeof(double)));
+    if (!c->d_startvals) NV_HIP(c, ctx_alloc(c, (void **)&c->d_startvals, NV_MAXS * sizeof(double)));
     NV_HIP(c, hipMemcpyAsync(c->d_startvals, vals.data(), op.ns * sizeof(double), hipMemcpyHostToDevice, c->stream));
     NV_HIP(c, nv::launch_fill_start(dst, op.D, (int)op.ns, c->d_startvals, c->stream));
     return NV_OK;
@@ -777,7 +809,7 @@ int32_t nv_start_vector(nv_ctx *c, double *q) {
     NV_HIP(c, hipSetDevice(c->device));
     const size_t bytes = (size_t)c->op.N * sizeof(double);
     double *tmp = nullptr;
-    NV_HIP(c, hipMalloc(&tmp, bytes));
+    NV_HIP(c, ctx_alloc(c, (void **)&tmp, bytes));
     int32_t rc = build_start(c, tmp);
     if (rc == NV_OK && q) {
         hipError_t e = hipMemcpyAsync(q, tmp, bytes, hipMemcpyDeviceToHost, c->stream);
@@ -829,7 +861,7 @@ int32_t nv_lanczos_init(nv_ctx *c, const nv_lanczos_opts *o) {
         release_lanczos(c);
         st.nslots = keep ? o->niter + 2 : 3;
         auto alloc = [&](size_t bytes, void **p) -> hipError_t {
-            hipError_t e = hipMalloc(p, bytes);
+            hipError_t e = ctx_alloc(c, p, bytes);
             if (e == hipSuccess) c->lz_allocs.push_back(*p);
             return e;
         };
@@ -885,8 +917,6 @@ int32_t nv_lanczos_init(nv_ctx *c, const nv_lanczos_opts *o) {
         NV_HIP(c, ensure_z2(c, nv::hv2_scratch_bytes(c->dev, o->prec)));
         st.z2 = c->z2;
     }
-    // (last, after what the run cannot do without)
-    if (!st.yt && !jit && use_fb(c, o->prec)) st.yt = alloc_slab(c, o->prec, c->lz_allocs);
     // start vector in the slot of iteration 1, beta(0) = |start|
     double *s1 = st.V + (1 % st.nslots) * N;
     int32_t rc = build_start(c, s1);
@@ -897,6 +927,8 @@ int32_t nv_lanczos_init(nv_ctx *c, const nv_lanczos_opts *o) {
         NV_HIP(c, hipMemsetAsync(c->cp, 0, (size_t)N * sizeof(double), c->stream));
         NV_HIP(c, hipMemcpyAsync(c->cp + N, s1, (size_t)N * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
     }
+    // (last, after what the run cannot do without, the scratch of its start vector among it)
+    if (!st.yt && !jit && use_fb(c, o->prec)) st.yt = alloc_slab(c, o->prec, c->lz_allocs);
     c->lz_ready = true;
     c->last_iter = 0;
     c->next_update = 1;
@@ -1425,7 +1457,7 @@ int32_t nv_identify_roots(nv_ctx *c, int64_t n, const double *alpha, const doubl
     const double *vec = (const double *)vecs.b.p;
     std::vector<void *> tmp;
     auto alloc = [&](size_t bytes, void **p) -> hipError_t {
-        hipError_t er = hipMalloc(p, bytes);
+        hipError_t er = ctx_alloc(c, p, bytes);
         if (er == hipSuccess) tmp.push_back(*p);
         return er;
     };
@@ -1749,7 +1781,7 @@ int32_t nv_lanczos_adjoint(nv_ctx *c, int64_t n, const double *abar, const doubl
     NV_HIP(c, hipMemcpy(beta_h.data(), c->st.beta, (niter + 3) * sizeof(double), hipMemcpyDeviceToHost));
     std::vector<void *> tmp;
     auto alloc = [&](size_t bytes, void **p) -> hipError_t {
-        hipError_t er = hipMalloc(p, bytes);
+        hipError_t er = ctx_alloc(c, p, bytes);
         if (er == hipSuccess) tmp.push_back(*p);
         return er;
     };
@@ -1830,7 +1862,7 @@ static int32_t spectrum_common(nv_ctx *c, int64_t n, const double *alpha, const 
     const double *vec = (const double *)vecs.b.p;
     std::vector<void *> tmp;
     auto alloc = [&](size_t bytes, void **p) -> hipError_t {
-        hipError_t er = hipMalloc(p, bytes);
+        hipError_t er = ctx_alloc(c, p, bytes);
         if (er == hipSuccess) tmp.push_back(*p);
         return er;
     };
@@ -1898,7 +1930,7 @@ int32_t nv_krylov_gradient(nv_ctx *c, int64_t n, const double *tbar, double *g_o
     const int64_t jc = std::min<int64_t>(K, nv::kRitzChunk);
     std::vector<void *> tmp;
     auto alloc = [&](size_t bytes, void **p) -> hipError_t {
-        hipError_t er = hipMalloc(p, bytes);
+        hipError_t er = ctx_alloc(c, p, bytes);
         if (er == hipSuccess) tmp.push_back(*p);
         return er;
     };
@@ -2020,7 +2052,7 @@ int32_t nv_convolve(nv_ctx *c, int64_t n, const double *x, const double *y, int6
     NV_HIP(c, hipSetDevice(c->device));
     double *d = nullptr;
     const size_t bytes = (size_t)(2 * n + 2 * ng + nv::convolve_parts(ng)) * sizeof(double);
-    NV_HIP(c, hipMalloc(&d, bytes));
+    NV_HIP(c, ctx_alloc(c, (void **)&d, bytes));
     double *dx = d, *dy = d + n, *dg = d + 2 * n, *de = d + 2 * n + ng, *dp = d + 2 * n + 2 * ng;
     hipError_t e = hipMemcpyAsync(dx, x, n * 8, hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(dy, y, n * 8, hipMemcpyHostToDevice, c->stream);
@@ -2306,8 +2338,8 @@ hipError_t batch_tiles(nv_batch *b, int bs) {
     if (b->tile0_d) hipFree(b->tile0_d);
     b->tiles_d = nullptr;
     b->tile0_d = nullptr;
-    hipError_t e = hipMalloc(&b->tiles_d, t.size() * sizeof(nv::BatchTile));
-    if (e == hipSuccess) e = hipMalloc(&b->tile0_d, t0.size() * sizeof(int32_t));
+    hipError_t e = nv::device_alloc((void **)&b->tiles_d, t.size() * sizeof(nv::BatchTile));
+    if (e == hipSuccess) e = nv::device_alloc((void **)&b->tile0_d, t0.size() * sizeof(int32_t));
     if (e == hipSuccess) e = hipMemcpy(b->tiles_d, t.data(), t.size() * sizeof(nv::BatchTile), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(b->tile0_d, t0.data(), t0.size() * sizeof(int32_t), hipMemcpyHostToDevice);
     b->d.tiles = b->tiles_d;
@@ -2377,10 +2409,10 @@ int32_t nv_batch_create(const nv_problem *probs, int64_t count, int32_t device, 
     };
     hipError_t e = hipSetDevice(device);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipMalloc(&b->ops_d, ops.size() * sizeof(NvOpDev));
-    if (e == hipSuccess) e = hipMalloc(&b->voff_d, b->voff.size() * sizeof(int64_t));
-    if (e == hipSuccess) e = hipMalloc(&b->loff_d, b->loff.size() * sizeof(int64_t));
-    if (e == hipSuccess) e = hipMalloc(&b->iter_d, sizeof(int64_t));
+    if (e == hipSuccess) e = nv::device_alloc((void **)&b->ops_d, ops.size() * sizeof(NvOpDev));
+    if (e == hipSuccess) e = nv::device_alloc((void **)&b->voff_d, b->voff.size() * sizeof(int64_t));
+    if (e == hipSuccess) e = nv::device_alloc((void **)&b->loff_d, b->loff.size() * sizeof(int64_t));
+    if (e == hipSuccess) e = nv::device_alloc((void **)&b->iter_d, sizeof(int64_t));
     if (e == hipSuccess) e = hipMemcpy(b->ops_d, ops.data(), ops.size() * sizeof(NvOpDev), hipMemcpyHostToDevice);
     if (e == hipSuccess)
         e = hipMemcpy(b->voff_d, b->voff.data(), b->voff.size() * sizeof(int64_t), hipMemcpyHostToDevice);
@@ -2446,7 +2478,7 @@ int32_t nv_batch_init(nv_batch *b, int64_t niter, int32_t prec) {
         int64_t maxtiles = 0;
         for (nv_ctx *c : b->ctx) maxtiles += (c->op.D + 63) / 64;  // the smallest tile size
         auto alloc = [&](size_t bytes, void **p) -> hipError_t {
-            hipError_t er = hipMalloc(p, bytes);
+            hipError_t er = nv::device_alloc(p, bytes);
             if (er == hipSuccess) b->run_allocs.push_back(*p);
             return er;
         };
@@ -2484,7 +2516,7 @@ int32_t nv_batch_init(nv_batch *b, int64_t niter, int32_t prec) {
         if (b->starts_d) hipFree(b->starts_d);
         b->starts_d = nullptr;
         b->starts_cap = 0;
-        NV_BHIP(b, hipMalloc(&b->starts_d, pts.size() * sizeof(nv::BatchStart)));
+        NV_BHIP(b, nv::device_alloc((void **)&b->starts_d, pts.size() * sizeof(nv::BatchStart)));
         b->starts_cap = pts.size();
     }
     if (!pts.empty()) {

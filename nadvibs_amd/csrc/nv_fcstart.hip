@@ -242,7 +242,7 @@ hipError_t build_fc_start(const Operator &op, const NvOpDev &dev, double *dst, h
     const int64_t D = op.D;
     std::vector<void *> tmp;
     auto up = [&](const void *src, size_t bytes, void **out) -> hipError_t {
-        hipError_t e = hipMalloc(out, bytes);
+        hipError_t e = device_alloc(out, bytes);
         if (e != hipSuccess) return e;
         tmp.push_back(*out);
         return hipMemcpyAsync(*out, src, bytes, hipMemcpyHostToDevice, s);
@@ -260,12 +260,12 @@ hipError_t build_fc_start(const Operator &op, const NvOpDev &dev, double *dst, h
     double *C[3] = {nullptr, nullptr, nullptr}, *part = nullptr, *sc = nullptr;
     const unsigned g = (unsigned)((D + 255) / 256);
     for (int k = 0; k < 3 && e == hipSuccess; ++k) {
-        e = hipMalloc((void **)&C[k], D * sizeof(double));
+        e = device_alloc((void **)&C[k], D * sizeof(double));
         if (e == hipSuccess) tmp.push_back(C[k]);
     }
-    if (e == hipSuccess) e = hipMalloc((void **)&part, g * sizeof(double));
+    if (e == hipSuccess) e = device_alloc((void **)&part, g * sizeof(double));
     if (e == hipSuccess) tmp.push_back(part);
-    if (e == hipSuccess) e = hipMalloc((void **)&sc, op.ns * sizeof(double));
+    if (e == hipSuccess) e = device_alloc((void **)&sc, op.ns * sizeof(double));
     if (e == hipSuccess) tmp.push_back(sc);
     // C(0) = 1; every other entry is written before it is read
     const double one = 1.0;

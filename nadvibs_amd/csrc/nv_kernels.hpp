@@ -9,6 +9,10 @@ namespace nv {
 
 constexpr int kBlock = 256;
 
+// hipMalloc on the current device that first frees what is only kept there for later calls when the
+// memory is short (nv_api.hip).
+hipError_t device_alloc(void **p, size_t bytes);
+
 // Device-side state of one Lanczos run.  Vector q_j lives in slot j % nslots
 // of V (nslots = niter+2 when the Krylov basis is kept, else 3); the slot of
 // iteration i+1 holds the unnormalised residual until update_lanczos(i+1).

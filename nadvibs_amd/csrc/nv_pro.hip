@@ -609,7 +609,7 @@ hipError_t pro_init(ProState &ps, const nv_lanczos_opts &o, const Operator &op, 
     ps.nchunks = p.nchunks;
     ps.jcap = p.jcap;
     auto alloc = [&](size_t bytes, void **ptr) -> hipError_t {
-        hipError_t e = hipMalloc(ptr, bytes);
+        hipError_t e = device_alloc(ptr, bytes);
         if (e == hipSuccess) allocs.push_back(*ptr);
         return e;
     };

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 import torch
 
+from nadvibs_amd._lib import NvError
 from nadvibs_amd.batch import Batch
 from nadvibs_amd.engine import Engine
 from nadvibs_amd.synth import make_problem
@@ -62,3 +63,52 @@ def test_solves_at_once_on_one_context():
         for t in threads:
             t.join()
     assert not wrong, wrong
+
+
+def test_a_failed_allocation_takes_back_the_workspace():
+    """What is kept for the next solve goes before a call fails for want of memory, and the context
+    works on."""
+    a, b = _tridiagonal(1600, 5)
+    # 1.4e6 elements: a basis of 10^6 of them is 11 TB
+    with Engine(make_problem(3, [12, 10, 10, 8, 8, 6], 2, (500, 3000), 200.0, 40.0, 20.0, seed=4)) as eng:
+        want = eng.ritz(a, b)
+        torch.cuda.synchronize()
+        free0 = torch.cuda.mem_get_info()[0]
+        with pytest.raises(NvError):
+            eng.lanczos_init(niter=1000000, savevecs=True)
+        gained = torch.cuda.mem_get_info()[0] - free0
+        print(f"given back: {gained >> 20} MB", flush=True)
+        assert gained >= 40 * 1600 * 1600 - (8 << 20)
+        for got, ref in zip(eng.ritz(a, b), want):
+            assert np.array_equal(got, ref)
+        eng.lanczos_init(niter=10)
+        eng.run(1, 10)
+        assert np.all(np.isfinite(eng.coefficients()[0]))
+
+
+@pytest.mark.parametrize("prec,tol", [("f64", 1e-11), ("f32", 5e-6)])
+def test_a_failed_allocation_takes_back_the_slab_buffer(prec, tol, monkeypatch):
+    """A run goes on without the slab buffer of its H*v when another call on its context needs the
+    memory.  Both forms sum the same at most 1,500 products a row: bounds as for the coefficients of
+    the slab pass against the step lists."""
+    for v in ("NV_HV_KERNEL", "NV_HV_FB"):
+        monkeypatch.delenv(v, raising=False)
+    p = make_problem(4, [8] * 7, 3, (400, 2500), 200.0, 60.0, 40.0, cubic=10.0, seed=7)
+    buffer = p.n * (8 if prec == "f64" else 4)
+    with Engine(p) as eng:
+        eng.lanczos_init(niter=12, prec=prec)
+        eng.run(1, 12)
+        want = eng.coefficients()[:2]
+        eng.lanczos_init(niter=12, prec=prec)
+        eng.run(1, 5)
+        eng.coefficients()
+        free0 = torch.cuda.mem_get_info()[0]
+        n = 400000  # 40 n^2 bytes: 6.4 TB
+        with pytest.raises(NvError):
+            eng.ritz(np.ones(n), np.ones(n + 1))
+        gained = torch.cuda.mem_get_info()[0] - free0
+        print(f"given back: {gained >> 20} MB of {buffer >> 20}", flush=True)
+        assert gained >= buffer - (8 << 20)
+        eng.run(6, 12)
+        for got, ref in zip(eng.coefficients()[:2], want):
+            assert np.max(np.abs(got - ref)) <= tol * np.max(np.abs(ref))
