@@ -2,8 +2,11 @@
 one before keeps its buffers and captured iterations, another shape replaces
 them, and coefficients read between the parts of a run are those of the
 iterations so far: always the numbers of a batch that runs once."""
+import time
+
 import numpy as np
 import pytest
+import torch
 
 from nadvibs_amd.batch import Batch
 from nadvibs_amd.synth import make_problem
@@ -52,3 +55,50 @@ def test_repeated_runs(shapes, prec):
         bt.init(18, prec)
         bt.run()
         assert np.array_equal(_all(bt, len(probs), 18), want[18])
+
+
+def test_watching_one_problem_of_a_long_run():
+    """Reading one problem between the parts of a run costs what it holds, not what the batch does
+    (64 problems of 20,000 iterations: 20 MB): at most five times the same read from a batch of one,
+    where a copy of the batch would take more than fifty; and every problem read after the same part
+    has the same numbers whether it came alone or with the others."""
+    p = make_problem(2, [6, 6, 5], 2, (500, 3000), 250.0, 60.0, 40.0, seed=70)
+    times = {}
+    for count in (1, 64):
+        with Batch([p] * count) as bt:
+            bt.init(20000, "f64")
+            bt.run(1, 8)
+            n, best = 8, np.inf
+            for _ in range(12):
+                bt.run(n + 1, n + 1)
+                n += 1
+                torch.cuda.synchronize()
+                t0 = time.perf_counter()
+                one = bt.coefficients(count - 1, n)
+                best = min(best, time.perf_counter() - t0)
+            times[count] = best
+            # the iterations of one problem are those of every other
+            for k in list(range(count)) + list(range(count)):
+                for got, want in zip(bt.coefficients(k, n), one):
+                    assert np.array_equal(got, want)
+    print(f"one read: {times[1] * 1e6:.0f} us of one problem, {times[64] * 1e6:.0f} us of 64", flush=True)
+    assert times[64] <= 5.0 * times[1]
+
+
+def test_reads_on_both_sides_of_the_copy_of_all():
+    """Forty problems of 2,000 iterations are 1.3 MB: the first reads come one by one, the rest from
+    one copy, in any order and again."""
+    probs = [make_problem(2, [5 + k % 3, 6, 4], 2, (500, 3000), 250.0, 60.0, 40.0, seed=k) for k in range(40)]
+    with Batch(probs) as bt:
+        bt.init(2000, "f64")
+        bt.run(1, 20)
+        order = np.random.default_rng(1).permutation(40)
+        got = {int(k): bt.coefficients(int(k), 20) for k in order}
+        again = {k: bt.coefficients(k, 20) for k in range(40)}
+    for k, prob in enumerate(probs):
+        with Batch([prob]) as bt:
+            bt.init(2000, "f64")
+            bt.run(1, 20)
+            want = bt.coefficients(0, 20)
+        for g in (got[k], again[k]):
+            assert np.array_equal(g[0], want[0]) and np.array_equal(g[1], want[1])
