@@ -2270,7 +2270,11 @@ struct nv_batch {
     size_t starts_cap = 0;
     std::vector<void *> allocs, run_allocs;
     size_t lds_hv = 0, lds_step = 0;
-    bool tuned = false;  // nv_batch_tune has chosen rows, tiles and form
+    // what nv_batch_tune chose for runs in FP64 and in FP32: rows per tile, rows per thread, kernel form
+    struct Form {
+        bool tuned = false;
+        int bs = 256, rows = 2, steps = 0;
+    } form[2];
     bool rows4 = false;  // lds_hv holds the digits of four rows per thread (FP32 shaped H*v)
     hipGraphExec_t graph = nullptr;
     hipGraphExec_t graph16 = nullptr;  // 16 iterations
@@ -2559,12 +2563,16 @@ int32_t nv_batch_init(nv_batch *b, int64_t niter, int32_t prec) {
     // four rows per thread (FP32, shaped form) where their digits fit in 64 KB of LDS
     b->rows4 = prec != NV_PREC_F64 && b->d.shaped[1] != 0 && lds4 <= 65536;
     if (b->rows4) b->lds_hv = lds4;
-    int rows = b->d.rows;
+    // A choice of the tuner holds for runs of the precision it was made in (FP64 knows one row per
+    // thread only, and would leave it to FP32 runs after it).
+    const nv_batch::Form &form = b->form[prec == NV_PREC_F64 ? 0 : 1];
+    if (form.bs != b->bs) NV_BHIP(b, batch_tiles(b, form.bs));
+    int rows = form.rows;
     // FP32 rows per thread of the shaped form, where nv_batch_tune has not chosen: more rows share a
     // term's descriptors and keep more loads in flight, fewer leave more waves.  17 iterations at 1,
     // 2, 4 rows per thread: 22,400 tiles 12.9, 10.6, 9.9 ms; 3,370 tiles 2.47, 2.18, 2.16; 1,860
     // tiles 1.65, 1.52, 1.67; 640 tiles 1.12, 1.16, 1.31.
-    if (!b->tuned && prec != NV_PREC_F64 && b->d.shaped[1])
+    if (!form.tuned && prec != NV_PREC_F64 && b->d.shaped[1])
         rows = b->d.T >= 4096 && b->rows4 ? 4 : b->d.T >= 1024 ? 2 : 1;
     if (const char *r = std::getenv("NV_BATCH_ROWS")) {
         const int v = std::atoi(r);
@@ -2574,8 +2582,9 @@ int32_t nv_batch_init(nv_batch *b, int64_t niter, int32_t prec) {
             return bfail(b, NV_ERR_ARG, "four rows per thread need the shaped form, 256-row tiles and LDS room");
         rows = v;
     }
-    if (rows != b->d.rows) batch_release_graphs(b);  // captured iterations name the kernel
+    if (rows != b->d.rows || form.steps != b->d.steps) batch_release_graphs(b);  // captured iterations name the kernel
     b->d.rows = rows;
+    b->d.steps = form.steps;
     b->ready = true;
     return NV_OK;
 }
@@ -2719,7 +2728,7 @@ int32_t nv_batch_tune(nv_batch *b, char *report, int64_t len) {
     if (e == hipSuccess) e = batch_tiles(b, best.bs);
     b->d.rows = best.rows;
     b->d.steps = best.steps;
-    b->tuned = true;
+    if (e == hipSuccess) b->form[b->prec == NV_PREC_F64 ? 0 : 1] = {true, best.bs, best.rows, best.steps};
     // alpha(1) of the timing launches is recomputed by the first iteration
     if (e == hipSuccess) e = hipMemsetAsync(b->d.alpha, 0, (size_t)b->ctx.size() * b->d.ld * sizeof(double), b->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(b->stream);

@@ -102,3 +102,28 @@ def test_reads_on_both_sides_of_the_copy_of_all():
             want = bt.coefficients(0, 20)
         for g in (got[k], again[k]):
             assert np.array_equal(g[0], want[0]) and np.array_equal(g[1], want[1])
+
+
+def test_tuning_holds_for_the_precision_it_was_made_in():
+    """A run takes the form that was tuned in its own precision, or the default one: the sums of its
+    workgroups, and so the last bits, are those of a batch that knew no other precision."""
+    probs = _probs(SHAPES["two rows"])
+    n = 18
+
+    def run(bt, prec):
+        bt.init(n, prec)
+        bt.run()
+        return _all(bt, len(probs), n)
+
+    fresh = {}
+    for prec in ("f64", "f32"):
+        with Batch(probs) as bt:
+            fresh[prec] = run(bt, prec)
+    for first, other in (("f64", "f32"), ("f32", "f64")):
+        with Batch(probs) as bt:
+            bt.init(n, first)
+            print(bt.tune(), flush=True)
+            bt.run()
+            tuned = _all(bt, len(probs), n)
+            assert np.array_equal(run(bt, other), fresh[other])
+            assert np.array_equal(run(bt, first), tuned)
