@@ -58,7 +58,7 @@ struct nv_ctx {
     std::string jit_log;
     float *hx32 = nullptr;
     void *yt[2] = {nullptr, nullptr};     // slab pass of a standalone fast-block H*v, FP64 and FP32 (in allocs)
-    bool yt_asked[2] = {false, false};    // its memory was asked for (once: a later call may be captured)
+    bool yt_short[2] = {false, false};    // there was no memory for it when it was last asked for
     double *hx64i = nullptr;              // interleaved FP64 copy of a standalone H*v input (two-pass form)
     void *z2 = nullptr;                   // channel scratch of the two-pass H*v
     size_t z2_bytes = 0;
@@ -704,8 +704,16 @@ static hipError_t hv_apply(nv_ctx *c, int32_t prec, const double *x, double *y, 
         if (e != hipSuccess) return e;
         const int k32 = prec == NV_PREC_F32;
         void *&yt = c->yt[k32];
-        if (!c->yt_asked[k32]) yt = alloc_slab(c, prec, c->allocs);
-        c->yt_asked[k32] = true;
+        if (!yt && c->dev.slab.on) {
+            // (a captured call allocates nothing: it takes every step in the sweep)
+            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+            e = hipStreamIsCapturing(s, &cap);
+            if (e != hipSuccess) return e;
+            if (cap == hipStreamCaptureStatusNone) {
+                yt = alloc_slab(c, prec, c->allocs);
+                c->yt_short[k32] = !yt;
+            }
+        }
         return nv::launch_hv_fb_full(c->dev, prec, x, xin, yt, y, s);
     }
     if (use_hv2(c, prec)) {
