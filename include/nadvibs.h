@@ -394,8 +394,9 @@ int32_t nv_hv_flops(const nv_ctx *ctx, int64_t *flops);
  * pair of HIP events on the context's stream.  Overwrites alpha(1). */
 int32_t nv_profile_hv(nv_ctx *ctx, int64_t launches, double *avg_us);
 /* Which H*v kernel serves precision prec: the operator-specialised one
- * (compiled at run time, on first use) or the generic one, as text.  The
- * environment variable NV_HV_KERNEL=generic selects the generic kernel. */
+ * (compiled at run time, on first use) or the generic one, with its form and
+ * the passes it takes, as text (up to 400 characters).  The environment
+ * variable NV_HV_KERNEL=generic selects the generic kernel. */
 int32_t nv_hv_kernel_info(nv_ctx *ctx, int32_t prec, char *buf, int64_t len);
 
 #ifdef __cplusplus

@@ -439,8 +439,11 @@ int32_t nv_create(const nv_problem *prob, int32_t device, nv_ctx **out) {
     // of a cubic operator): 88.5M elements, 560 steps, 10.6 -> 8.0 ms (FP32) and 23.0 -> 17.4 ms
     // (FP64); two states, 3.6M rows, 220 steps: 1,091 -> 911 us and 1,125 -> 1,117 us; with 120 or 56
     // the extra pass over the vectors costs what the steps do (three states, 1.3M rows, FP64: 406
-    // against 441 us; four, 1.4M rows: 361 against 426 us).  NV_HV_FB=1 takes it always.
-    if (d.fb.on && op.slab && (op.slab_steps >= 200 || d.fb_min_bytes == 0)) {
+    // against 441 us; four, 1.4M rows: 361 against 426 us).  NV_HV_FB=1 takes it always, NV_HV_SLAB=1
+    // too, and NV_HV_SLAB=0 never.
+    const char *slab = std::getenv("NV_HV_SLAB");
+    const bool slab_on = slab ? std::strcmp(slab, "0") != 0 : op.slab_steps >= 200 || d.fb_min_bytes == 0;
+    if (d.fb.on && op.slab && slab_on) {
         NvSlabDev &l = d.slab;
         l.gl = op.slab_gl;
         l.nl = op.slab_nl;
@@ -989,23 +992,45 @@ int32_t nv_hv_kernel_info(nv_ctx *c, int32_t prec, char *buf, int64_t len) {
     NV_HIP(c, hipSetDevice(c->device));
     const nv::JitKernels *k = ensure_jit(c, prec);
     std::string t = k ? "operator-specialised (hiprtc)"
-                      : (std::string(nv::hv_shaped(c->dev, prec) ? "generic shaped" : "generic step-table") +
-                         (c->jit_log.empty() ? std::string() : ": " + c->jit_log));
+                      : std::string(nv::hv_shaped(c->dev, prec) ? "generic shaped" : "generic step-table");
+    char x[256];
     if (!k && use_fb(c, prec)) {
-        char fbs[160];
-        std::snprintf(fbs, sizeof fbs,
+        std::snprintf(x, sizeof x,
                       "generic fast-block (%d rows per wave over modes %d..%lld; slow steps scalar, fast steps "
                       "through LDS)",
                       (int)c->dev.fb.P, (int)c->dev.fb.mf, (long long)c->op.M - 1);
-        t = fbs;
-    } else if (!k && use_hv2(c, prec))
+        t = x;
+        const NvSlabDev &l = c->dev.slab;
+        if (l.on) {
+            std::snprintf(x, sizeof x, ", degree-three slow steps in a slab pass (modes %d..%d in LDS)", (int)l.gl,
+                          (int)(l.gl + l.nl - 1));
+            t += x;
+            if (l.kl > 0) {
+                std::snprintf(x, sizeof x, " and a leading pass (modes 0..%d)", (int)l.kl - 1);
+                t += x;
+            }
+            // (the buffer of a run is asked for at its start, that of a standalone H*v at the first call)
+            const bool run = c->lz_ready && c->opts.prec == prec && !c->st.yt;
+            const bool alone = c->yt_short[prec == NV_PREC_F32];
+            if (run || alone)
+                t += std::string(" [no memory for the slab buffer of ") +
+                     (run && alone ? "the run and of the standalone H*v" : run ? "the run" : "the standalone H*v") +
+                     ": all steps in the sweep]";
+        } else if (c->op.slab) {
+            t += ", all slow steps in the sweep";
+        }
+    } else if (!k && use_hv2(c, prec)) {
         t = std::string("generic two-pass (modes 0 and 1 split off; coupling products on ") +
             (prec == NV_PREC_F32 && c->dev.hv2.mfma ? "MFMA" : "the VALU") + ")";
-    else if (!k && nv::hv_shaped(c->dev, prec)) {
-        char extra[96];
-        std::snprintf(extra, sizeof extra, " [%s; steps inside the basis %.6f]",
-                      nv::hv_shaped_skip(c->dev, prec) ? "skip form" : "plain form", c->op.step_valid);
-        t += extra;
+    } else if (!k) {
+        const int waves = nv::hv_split_waves(c->dev, prec);
+        if (waves > 1) t += ", a row's terms shared over " + std::to_string(waves) + " waves";
+        if (!c->jit_log.empty()) t += ": " + c->jit_log;
+        if (nv::hv_shaped(c->dev, prec)) {
+            std::snprintf(x, sizeof x, " [%s; steps inside the basis %.6f]",
+                          nv::hv_shaped_skip(c->dev, prec) ? "skip form" : "plain form", c->op.step_valid);
+            t += x;
+        }
     }
     std::snprintf(buf, (size_t)len, "%s", t.c_str());
     return NV_OK;

@@ -1166,9 +1166,11 @@ static bool hv_split(const NvOpDev &op, int prec, int rows) {
            hv_lds_bytes(op, 0) + (size_t)(kSplitWaves - 1) * op.ns * 64 * sizeof(double) <= 65536;
 }
 static unsigned hv_split_blocks(const NvOpDev &op) { return (unsigned)((op.D + 63) / 64); }
+int hv_split_waves(const NvOpDev &op, int prec) {
+    return hv_shaped(op, prec) && !hv_shaped_skip(op, prec) && hv_split(op, prec, kSplitRows) ? kSplitWaves : 1;
+}
 static bool hv_split_iter(const NvOpDev &op, int prec, const LzState &st) {
-    return (prec == 0 ? (void *)st.v64i : st.vlo) && hv_shaped(op, prec) && !hv_shaped_skip(op, prec) &&
-           hv_split(op, prec, kSplitRows);
+    return (prec == 0 ? (void *)st.v64i : st.vlo) && hv_split_waves(op, prec) > 1;
 }
 
 template <int NS>

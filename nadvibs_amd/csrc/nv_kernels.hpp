@@ -64,6 +64,8 @@ bool hv_shaped(const NvOpDev &op, int prec);
 // Whether the shaped iteration H*v of precision prec points the loads of
 // out-of-basis steps outside the vector (vector above op.skip_min_bytes).
 bool hv_shaped_skip(const NvOpDev &op, int prec);
+// Waves over which the iteration kernel of the shaped form shares the terms of a row (1: a row per thread).
+int hv_split_waves(const NvOpDev &op, int prec);
 // Two-pass H*v (NvHv2Dev): whether it serves precision prec (tables built,
 // vector at least op.hv2_min_bytes), its channel scratch, and the number of
 // alpha partials the iteration H*v then writes.

@@ -267,8 +267,8 @@ class Engine:
 
     def hv_kernel(self, prec="f64"):
         """Which H*v kernel serves `prec` (compiles it on first use)."""
-        buf = ctypes.create_string_buffer(256)
-        self._check(self.lib.nv_hv_kernel_info(self.h, _lib.PREC[prec], buf, 256))
+        buf = ctypes.create_string_buffer(512)
+        self._check(self.lib.nv_hv_kernel_info(self.h, _lib.PREC[prec], buf, 512))
         return buf.value.decode()
 
     def convolve(self, x, y, grid, sigma):

@@ -93,3 +93,32 @@ def test_shared_terms_fp32(case, monkeypatch):
         got = results(eng, "f32")
     for tol, g, r in zip((2e-6, 5e-6, 5e-6), got, ref):
         assert np.max(np.abs(g - r)) <= tol * np.max(np.abs(r))
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"{c[0]}x{'-'.join(map(str, c[1]))}o{c[2]}")
+def test_shared_terms_are_reported(case, monkeypatch):
+    """Which of the FP64 operators above share a row's terms in their iterations: 512 to 262,144 rows."""
+    for v in ("NV_HV_KERNEL", "NV_HV_FB"):
+        monkeypatch.delenv(v, raising=False)
+    ns, nf, ordr, offe, quirks = case
+    p = make_problem(ns, nf, ordr, (400, 2500), 200.0, 60.0, 40.0, cubic=10.0, seed=len(nf), quirks=quirks,
+                     offdiag_even=offe)
+    rows = int(np.prod(nf))
+    with Engine(p) as eng:
+        info = eng.hv_kernel("f64")
+        assert info.startswith("generic shaped"), info
+        assert ("terms shared over 4 waves" in info) == (512 <= rows <= 262144), info
+
+
+@pytest.mark.parametrize("case", MANY, ids=lambda c: f"{c[0]}x{'-'.join(map(str, c[1]))}")
+def test_shared_terms_fp32_are_reported(case):
+    ns, nf, offe, quirks = case
+    p = make_problem(ns, nf, 3, (400, 2500), 200.0, 60.0, 40.0, cubic=10.0, seed=len(nf), quirks=quirks,
+                     offdiag_even=offe)
+    with Engine(p) as eng:
+        eng.select_hv_kernel(True)
+        assert "terms shared over 4 waves" in eng.hv_kernel("f32")
+    few = make_problem(3, [8, 8, 8], 2, (400, 2500), 200.0, 60.0, 40.0, seed=1)
+    with Engine(few) as eng:
+        eng.select_hv_kernel(True)
+        assert "waves" not in eng.hv_kernel("f32")
