@@ -21,6 +21,10 @@
 #include "nv_pro.hpp"
 #include "nv_workspace.hpp"
 
+// Most partials that the kernels after a sum add up themselves in captured iterations (see
+// enqueue_folded_batch); half of what the partials buffer always holds.
+constexpr int kFoldMax = 4096;
+
 struct nv_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -49,6 +53,7 @@ struct nv_ctx {
     // [2] re-orthogonalisation with the exact overlap check
     hipGraphExec_t graphs[4] = {nullptr, nullptr, nullptr, nullptr};  // kinds 0-2, and kIterBatch of kind 0
     hipGraphExec_t graph = nullptr;
+    int fold_max = kFoldMax;
 
     // operator-specialised H*v kernels per precision (F64, F32)
     bool jit_on = true;
@@ -292,6 +297,8 @@ int32_t nv_create(const nv_problem *prob, int32_t device, nv_ctx **out) {
     {
         const char *k = std::getenv("NV_HV_KERNEL");
         c->jit_on = !(k && (std::strcmp(k, "generic") == 0 || std::strcmp(k, "steps") == 0));
+        if (const char *m = std::getenv("NV_FOLD_MAX"))
+            c->fold_max = std::max(0, std::min(kFoldMax, std::atoi(m)));
     }
     hipError_t e = hipSetDevice(device);
     if (e == hipSuccess) e = scratch_setup(device);
@@ -1172,7 +1179,7 @@ constexpr int64_t kIterBatch = 16;
 // odd).  The first iteration of a launch normalises with the stored beta, and
 // the last one's beta goes through the finishing kernel, so a launch starts
 // and ends in the state the per-call path leaves.
-constexpr int kFoldMax = 4096;
+// (NV_FOLD_MAX lowers the limit; 0: the finishing kernels always run.)
 
 // The iteration H*v without its alpha finish, and the partials it writes.
 static hipError_t launch_hv_iter_nofinish(nv_ctx *c, const nv::LzState &st) {
@@ -1184,7 +1191,7 @@ static int hv_iter_nparts(nv_ctx *c) {
     return ensure_jit(c, c->opts.prec) ? nv::hv_blocks(c->dev) : nv::hv_iter_parts(c->dev, c->opts.prec, c->st);
 }
 static bool fold_ok(nv_ctx *c) {
-    return hv_iter_nparts(c) <= kFoldMax && nv::hv_blocks(c->dev) <= kFoldMax;
+    return hv_iter_nparts(c) <= c->fold_max && nv::hv_blocks(c->dev) <= c->fold_max;
 }
 
 static hipError_t enqueue_folded_batch(nv_ctx *c) {
