@@ -16,6 +16,9 @@ namespace nv {
 constexpr int kSplit = 16;             // lanes per grid point
 constexpr int64_t kSplitGrid = 65536;  // 4096 workgroups of 16 points, 16 per CU
 
+// 1 / sigma, finite for the subnormal ones too: a stick at the grid point counts in full.
+__device__ __forceinline__ double inv_sigma(double sigma) { return fmin(1.0 / sigma, 1.7976931348623157e308); }
+
 // The sum over the sticks at gx; S lanes share it and all return it.  Sticks
 // go through LDS in tiles of kBlock; stick(j) gives (position, weight).
 template <int S, typename Stick>
@@ -42,7 +45,7 @@ __global__ __launch_bounds__(kBlock) void convolve_kernel(const double *x, const
                                                           const double *grid, int64_t ng, double sigma, double *env,
                                                           double *part) {
     const int64_t g = (int64_t)blockIdx.x * (kBlock / S) + threadIdx.x / S;
-    const double acc = gauss_sum<S>(g < ng ? grid[g] : 0.0, 1.0 / sigma, n, [&](int64_t j, double &sx, double &sy) {
+    const double acc = gauss_sum<S>(g < ng ? grid[g] : 0.0, inv_sigma(sigma), n, [&](int64_t j, double &sx, double &sy) {
         sx = x[j];
         sy = y[j];
     });
@@ -99,7 +102,7 @@ __global__ __launch_bounds__(kBlock) void spec_env_kernel(int64_t n, const doubl
                                                          double sigma, int64_t ng, const double *__restrict__ grid,
                                                          double *__restrict__ env) {
     const int64_t g = (int64_t)blockIdx.x * (kBlock / S) + threadIdx.x / S;
-    const double acc = gauss_sum<S>(g < ng ? grid[g] : 0.0, 1.0 / sigma, n, [&](int64_t i, double &sx, double &sy) {
+    const double acc = gauss_sum<S>(g < ng ? grid[g] : 0.0, inv_sigma(sigma), n, [&](int64_t i, double &sx, double &sy) {
         const double a = vec[i];
         sx = (theta[i] - ref) * c;
         sy = a * a;

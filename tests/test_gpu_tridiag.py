@@ -95,3 +95,18 @@ def test_envelope_sizes(eng, ng, n):
         ref += yi * np.exp(-0.5 * ((grid - xi) / 20.0) ** 2)
     # n products and sums, an exponential of an argument below 13 in magnitude
     np.testing.assert_allclose(env, ref / ref.max(), rtol=(n + 40) * np.finfo(float).eps)
+
+
+@pytest.mark.parametrize("ng", [3, 65537])
+def test_envelopes_of_the_narrowest_width(eng, ng):
+    """A width whose reciprocal overflows: the sticks on grid points alone, in full."""
+    rng = np.random.default_rng(2)
+    a, b = 0.1 + 0.05 * rng.standard_normal(20), 0.03 * np.ones(21)
+    _, it, _, _ = eng.ritz(a, b)
+    grid = np.linspace(0.0, 1e-3, ng)
+    for sigma in (1e-310, 5e-324, 1e-300):
+        want = np.zeros(ng)
+        want[0] = it[0]
+        assert np.array_equal(eng.spectrum(a, b, grid, sigma), want)
+        env = eng.convolve(np.array([0.0, 50.0]), np.array([2.0, 1.0]), grid, sigma)
+        assert np.array_equal(env, want != 0.0)
