@@ -1146,9 +1146,13 @@ bool hv_shaped_batch(const NvOpDev &op, int prec) { return prec == 0 ? shaped_st
 // three (cubic) 2467 -> 1802, 175,616 of two 1139 -> 1013, 262,144 of two
 // (cubic) 2781 -> 2528.  Two waves give less below 100,000 rows, eight lose
 // above (100,000 rows 1025 -> 943 us with four, 1010 with eight).  Standalone,
-// 460,800 rows of three states: 61.2 -> 56.6 us, cubic 298 -> 272.  Below
-// kSplitMinRows a run soon exhausts its Krylov space, after which every
-// rounding counts, and it keeps the sums of the batched kernels.
+// 460,800 rows of three states: 61.2 -> 56.6 us, cubic 298 -> 272.
+// kSplitMinRows is no line of speed: below it the shared form is the faster one
+// too (33 iterations, 64 rows of two states 462 against 404 us, 432 cubic rows
+// of three 1240 against 655).  But such a run soon exhausts its Krylov space,
+// after which rounding alone decides the coefficients, and it keeps the sums of
+// the batched kernels so that a problem gives the same numbers alone and in a
+// batch.
 // In FP32 it serves operators of kSplitTerms32 terms or more: those whose
 // steps are too many for the run-time compiled kernel.  17 iterations, cubic
 // operators of 9 and 10 modes: 1,536 rows of four states 2061 -> 720 us,

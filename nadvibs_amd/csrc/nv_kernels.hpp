@@ -158,7 +158,7 @@ struct TriWork {
     int64_t *rank = nullptr; // [n] number of cluster members (ia>0) before root i
 };
 // Smallest e^2 in TriWork::de (the host applies it): a zero one would stop the product form of the
-// Sturm sequence at an exactly zero pivot.
+// Sturm sequence at an exactly zero pivot (nv_tridiag.hip says what is left of that).
 constexpr double kTriMinE2 = 1e-200;
 int tri_grid_points(int64_t n);
 hipError_t launch_tridiag(int64_t n, const TriWork &w, hipStream_t s);

@@ -59,8 +59,14 @@ __device__ __forceinline__ double tri_div(double a, double d) {
 // where the quotient has a division.  The minors are rescaled by a power of
 // two every kSturm steps: |d - x| <= 2 and e^2 <= 1, so they grow by less than
 // 2.5 a step.  A zero minor counts as a nonnegative pivot followed by a
-// negative one, as there.  de is read with scalar loads, the next kSturm rows
-// while these are used.
+// negative one, as there.  That does not hold where several rows are exactly
+// decoupled (e^2 at its floor, kTriMinE2) and x is their common diagonal: the
+// minors can then underflow to zero between two rescalings, and the sign
+// changes after them are lost.  The search meets such an x only in the last
+// ulps of that diagonal's own roots; on the CPU, 96,000 roots of matrices with
+// repeated diagonals and zero couplings came within 1.7 * 2^-53 of the norm of
+// a bisection in 113-bit arithmetic.  de is read with scalar loads, the next
+// kSturm rows while these are used.
 constexpr int kSturm = 8;
 static_assert(kSturm <= kTriPad, "the prefetch reads kSturm rows past the matrix");
 
