@@ -47,6 +47,9 @@ struct nv_ctx {
     bool pro_loaded = false;     // nv_load_archive restored the re-orthogonalisation state
     int64_t next_update = 1;     // iteration expected by update_lanczos
     std::vector<void *> lz_allocs;
+    // held by the calls that launch the run's H*v or set the run up, so that a call of another thread
+    // does not take the slab buffer from under them
+    std::recursive_mutex run_mu;
     nv::ProState pro{};
 
     // graphs of one iteration: [0] plain, [1] with re-orthogonalisation,
@@ -265,10 +268,12 @@ bool valid_prec(int32_t p) { return p == NV_PREC_F64 || p == NV_PREC_F32 || p ==
 }  // namespace
 
 // Frees the slab buffer of the run, whose iterations then take every step in the sweep; whether
-// there was one to free.  Not where segments are recomputed from checkpoints: the recomputation is
-// checked bit for bit, and the two forms add in different orders.
+// there was one to free.  Not while another thread runs it, and not where segments are recomputed
+// from checkpoints: the recomputation is checked bit for bit, and the two forms add in different
+// orders.
 static bool drop_slab(nv_ctx *c) {
-    if (!c->st.yt || c->cp) return false;
+    std::unique_lock<std::recursive_mutex> lock(c->run_mu, std::try_to_lock);
+    if (!lock || !c->st.yt || c->cp) return false;
     if (hipStreamSynchronize(c->stream) != hipSuccess) return false;
     release_graphs(c);  // captured iterations name it
     c->lz_allocs.erase(std::find(c->lz_allocs.begin(), c->lz_allocs.end(), c->st.yt));
@@ -842,6 +847,7 @@ int32_t nv_start_vector(nv_ctx *c, double *q) {
 // ---- Lanczos --------------------------------------------------------------
 int32_t nv_lanczos_init(nv_ctx *c, const nv_lanczos_opts *o) {
     if (!c || !o) return NV_ERR_ARG;
+    std::lock_guard<std::recursive_mutex> run(c->run_mu);
     if (o->niter < 1) return fail(c, NV_ERR_ARG, "niter must be >= 1");
     if (!valid_prec(o->prec)) return fail(c, NV_ERR_ARG, "unknown precision");
     if (o->reorthog > 0 && nv::pro_decide_lds(o->niter) != 0)
@@ -976,6 +982,7 @@ int32_t nv_update_lanczos(nv_ctx *c, int64_t it) {
 int32_t nv_hv_iter(nv_ctx *c, int64_t it) {
     int32_t rc = check_iter(c, it);
     if (rc) return rc;
+    std::lock_guard<std::recursive_mutex> run(c->run_mu);
     if (it != c->next_update - 1) return fail(c, NV_ERR_STATE, "Hv called before update_lanczos");
     if (c->prof) {
         if (c->ev_used == c->ev.size()) {
@@ -1057,6 +1064,7 @@ int32_t nv_hv_flops(const nv_ctx *c, int64_t *flops) {
 
 int32_t nv_profile_hv(nv_ctx *c, int64_t launches, double *avg_us) {
     if (!c || !avg_us || launches < 1) return NV_ERR_ARG;
+    std::lock_guard<std::recursive_mutex> run(c->run_mu);
     if (!c->lz_ready || c->next_update < 2) return fail(c, NV_ERR_STATE, "update_lanczos(1) must come first");
     NV_HIP(c, hipSetDevice(c->device));
     const nv::JitKernels *k = ensure_jit(c, c->opts.prec);
@@ -1287,6 +1295,7 @@ static hipError_t iteration_graph(nv_ctx *c, int kind, hipGraphExec_t *out) {
 
 int32_t nv_lanczos_run(nv_ctx *c, int64_t iiter, int64_t niter) {
     if (!c) return NV_ERR_ARG;
+    std::lock_guard<std::recursive_mutex> run(c->run_mu);
     if (!c->lz_ready) return fail(c, NV_ERR_STATE, "nv_lanczos_init has not been called");
     if (iiter != c->next_update) return fail(c, NV_ERR_STATE, "run must start at the next iteration");
     if (niter > c->opts.niter) return fail(c, NV_ERR_ARG, "niter beyond the initialised run");

@@ -112,3 +112,39 @@ def test_a_failed_allocation_takes_back_the_slab_buffer(prec, tol, monkeypatch):
         eng.run(6, 12)
         for got, ref in zip(eng.coefficients()[:2], want):
             assert np.max(np.abs(got - ref)) <= tol * np.max(np.abs(ref))
+
+
+def test_a_run_keeps_its_slab_buffer_while_another_thread_lacks_memory(monkeypatch):
+    """One thread runs iterations, another fails again and again for want of memory: the run's launches
+    never lose the buffer they name.  Bounds as above."""
+    for v in ("NV_HV_KERNEL", "NV_HV_FB"):
+        monkeypatch.delenv(v, raising=False)
+    p = make_problem(4, [8] * 7, 3, (400, 2500), 200.0, 60.0, 40.0, cubic=10.0, seed=7)
+    n = 400000
+    diag, off = np.ones(n), np.ones(n + 1)
+    with Engine(p) as eng:
+        eng.lanczos_init(niter=12)
+        eng.run(1, 12)
+        want = eng.coefficients()[:2]
+        stop, failed = threading.Event(), []
+
+        def short():
+            while not stop.is_set():
+                try:
+                    eng.ritz(diag, off)
+                except NvError:
+                    failed.append(1)
+
+        t = threading.Thread(target=short)
+        t.start()
+        try:
+            for _ in range(6):
+                eng.lanczos_init(niter=12)
+                for i in range(1, 13, 3):
+                    eng.run(i, i + 2)
+                for got, ref in zip(eng.coefficients()[:2], want):
+                    assert np.max(np.abs(got - ref)) <= 1e-11 * np.max(np.abs(ref))
+        finally:
+            stop.set()
+            t.join()
+        assert failed
