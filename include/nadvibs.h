@@ -117,7 +117,8 @@ int32_t nv_term_counts(const nv_ctx *ctx, int64_t *out);
 /* y = H x for host arrays x, y of n doubles. */
 int32_t nv_hv(nv_ctx *ctx, int32_t prec, const double *x, double *y);
 /* y = H x for device arrays of n doubles, enqueued on `stream` (a
- * hipStream_t, NULL = the context's stream).  No host synchronisation. */
+ * hipStream_t, NULL = the context's stream, which does not wait for the
+ * default stream: hipStreamLegacy names that one).  No host synchronisation. */
 int32_t nv_hv_device(nv_ctx *ctx, int32_t prec, const double *x_dev,
                      double *y_dev, void *stream);
 
@@ -207,7 +208,7 @@ int32_t nv_get_lanczos_vector(nv_ctx *ctx, int64_t j, double *q);
  * and sign[i] = sign of v(1,i).  Runs on the context's device.  The device
  * workspace (40 n^2 bytes) is kept for the next solve, up to 512 MB in all for
  * the contexts of a device; it goes back with the last of them, and when an
- * eigensolve finds the memory short. */
+ * allocation of the library finds the memory short. */
 int32_t nv_ritz(nv_ctx *ctx, int64_t n, const double *alpha,
                 const double *beta, double *eval, double *inten, double *bji,
                 int32_t *sign);
@@ -325,7 +326,9 @@ int32_t nv_batch_init(nv_batch *b, int64_t niter, int32_t prec);
 int32_t nv_batch_tune(nv_batch *b, char *report, int64_t len);
 /* Iterations iiter..niter for every problem.  Asynchronous. */
 int32_t nv_batch_run(nv_batch *b, int64_t iiter, int64_t niter);
-/* alpha(1:n) and beta(0:n) of problem p (n = last iteration).  Synchronises. */
+/* alpha(1:n) and beta(0:n) of problem p (n = last iteration).  Synchronises.
+ * Reading every problem takes one copy for all of them; reading a few of a
+ * large batch copies theirs. */
 int32_t nv_batch_coefficients(nv_batch *b, int64_t p, double *alpha,
                               double *beta);
 /* The context of problem p (owned by the batch). */
